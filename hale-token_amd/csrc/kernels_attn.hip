@@ -17,14 +17,16 @@
 
 #include "hale_device.h"
 #include "kernels.h"
+#include "ordered_sum.h"
 
 namespace hale {
 
-constexpr int NORM_MAX = 8192;     // elements one RMSNorm work-group holds in LDS
+constexpr int NORM_MAX = ORDERED_MAX;  // elements of an RMSNorm row
 constexpr int HEAD_MAX = 1024;     // largest head_dim
 
 // inverse_rms (src/ops/norm.rs:25-28) of n values whose squares are in
-// sq[0, n) of LDS; every thread gets the scale.
+// sq[0, n) of LDS; every thread gets the scale.  One chain: for a head's
+// 64-128 values the lanes' scan (ordered_sum.h) would take as long.
 __device__ __forceinline__ float block_inverse_rms(const float* sq, int n, float eps, float* bcast) {
   if (threadIdx.x == 0) {
     const float s = lds_sum_in_order(sq, n, -0.0f);
@@ -36,23 +38,34 @@ __device__ __forceinline__ float block_inverse_rms(const float* sq, int n, float
 
 // One work-group per row: out = rms_norm(x + delta, w) with x updated to
 // x + delta first when delta is given (add_in_place, then rms_norm).  The
-// row and the weights are read once, all loads in flight together, and
-// stay in registers through the in-order sum of the squares.  (out may be x
+// row and the weights are read once, all loads in flight together, and stay
+// in registers through the in-order sum of the squares.  (out may be x
 // itself: every element is read before any is written.)
-constexpr int NORM_PER = NORM_MAX / 256;  // elements per thread
-
+//
+// Bound by latency: one load round trip, the ordered sum, one store.  The
+// squares go through LDS to become each lane's K consecutive values
+// (ordered_sum.h); K is the smallest of 4 .. 32 that covers the row, as
+// every unused K costs its predicated loads and chain steps.  One row of
+// 2048: 13.9 us with one chain of squares, 4.5 us so (a launch alone is
+// about 4); the norm and MoE of a Mixtral-shaped layer (rows of 4096) went
+// from 69.4 to 50.4 us.  The sum starts from +0: the reference's -0 start
+// shows only without values.
+template <int K>
 __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restrict__ delta,
                                                   const float* __restrict__ w, int n, float eps,
                                                   float* out) {
-  __shared__ __attribute__((aligned(16))) float sq[NORM_MAX];
-  __shared__ float bcast[1];
+  // 4 floats of padding every 32 keep the lanes' 16-byte reads at a stride
+  // of K floats off each other's banks
+  auto at = [](int i) { return i + (i >> 5) * 4; };
+  __shared__ __attribute__((aligned(16))) float sq[256 * K + 8 * K * 4];
+  __shared__ float part[ordered_lds(4)];
   float* xr = x + (size_t)blockIdx.x * n;
   const float* dr = delta ? delta + (size_t)blockIdx.x * n : nullptr;
   float* orow = out + (size_t)blockIdx.x * n;
   const int tid = threadIdx.x;
-  float xv[NORM_PER], wv[NORM_PER];
+  float xv[K], wv[K];
 #pragma unroll
-  for (int j = 0; j < NORM_PER; j++) {
+  for (int j = 0; j < K; j++) {
     const int i = tid + 256 * j;
     if (i < n) {
       xv[j] = xr[i];
@@ -60,24 +73,41 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
     }
   }
   if (dr) {
+    float dv[K];
 #pragma unroll
-    for (int j = 0; j < NORM_PER; j++) {
+    for (int j = 0; j < K; j++) {
+      const int i = tid + 256 * j;
+      if (i < n) dv[j] = dr[i];
+    }
+#pragma unroll
+    for (int j = 0; j < K; j++) {
       const int i = tid + 256 * j;
       if (i < n) {
-        xv[j] = xv[j] + dr[i];
+        xv[j] = xv[j] + dv[j];
         xr[i] = xv[j];
       }
     }
   }
 #pragma unroll
-  for (int j = 0; j < NORM_PER; j++) {
+  for (int j = 0; j < K; j++) {
     const int i = tid + 256 * j;
-    if (i < n) sq[i] = xv[j] * xv[j];
+    sq[at(i)] = i < n ? xv[j] * xv[j] : 0.0f;
   }
   __syncthreads();
-  const float scale = block_inverse_rms(sq, n, eps, bcast);
+  float v[K];
 #pragma unroll
-  for (int j = 0; j < NORM_PER; j++) {
+  for (int q = 0; q < K / 4; q++) {
+    const f32x4 t = *(const f32x4*)&sq[at(tid * K + 4 * q)];
+    v[4 * q] = t.x;
+    v[4 * q + 1] = t.y;
+    v[4 * q + 2] = t.z;
+    v[4 * q + 3] = t.w;
+  }
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float s = team_sum_in_order<K>(v, 0.0f, wave, 4, part);
+  const float scale = 1.0f / sqrtf(s / (float)n + eps);
+#pragma unroll
+  for (int j = 0; j < K; j++) {
     const int i = tid + 256 * j;
     if (i < n) orow[i] = xv[j] * scale * wv[j];
   }
@@ -566,7 +596,11 @@ hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t 
                            float eps, float* out, hipStream_t st) {
   if (rows == 0) return hipSuccess;
   if (n == 0 || n > (size_t)NORM_MAX || rows > 0x7fffffffu) return hipErrorInvalidValue;
-  return launch(k_rms_norm, (unsigned)rows, 256, 0, st, x, delta, w, (int)n, eps, out);
+  auto run = [&](auto kernel) { return launch(kernel, (unsigned)rows, 256, 0, st, x, delta, w, (int)n, eps, out); };
+  if (n <= 1024) return run(k_rms_norm<4>);
+  if (n <= 2048) return run(k_rms_norm<8>);
+  if (n <= 4096) return run(k_rms_norm<16>);
+  return run(k_rms_norm<32>);
 }
 
 hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {

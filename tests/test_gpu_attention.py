@@ -49,6 +49,42 @@ def test_rms_norm_reference_case_and_zero_row(ctx):
         H.rms_norm(ctx, np.zeros(8193, np.float32), np.ones(8193, np.float32), 1e-6)
 
 
+def squares_case(kind, n):
+    """Rows whose sum of squares meets the cases of the lanes' ordered sum:
+    every square half-way between two results (ties to even), values of all
+    binades, a first square of an exact power of two above all the rest,
+    zeros, a sum that becomes infinite, a NaN."""
+    g = np.random.default_rng(n * 31 + len(kind))
+    if kind == "normal":
+        return g.standard_normal(n).astype(np.float32)
+    if kind == "ties":
+        return (g.integers(0, 4, n) * np.where(g.random(n) < 0.1, 4096.0, 1.0)).astype(np.float32)
+    if kind == "binades":
+        return np.exp(g.uniform(-45, 40, n)).astype(np.float32)
+    if kind == "growing":
+        return np.exp(np.linspace(-43, 43, n)).astype(np.float32)
+    if kind == "sink":
+        x = (g.random(n) * 1e-3).astype(np.float32)
+        x[0] = 1.0
+        return x
+    if kind == "zeros":
+        return np.where(g.random(n) < 0.02, g.standard_normal(n), 0.0).astype(np.float32)
+    x = g.standard_normal(n).astype(np.float32)
+    x[n // 2] = 1e20 if kind == "inf" else np.nan
+    return x
+
+
+@pytest.mark.parametrize("kind", ["normal", "ties", "binades", "growing", "sink", "zeros", "inf", "nan"])
+def test_rms_norm_ordered_sum_edges(ctx, kind):
+    for n in (1, 3, 64, 65, 255, 256, 257, 1000, 1024, 1025, 2047, 2048, 2049, 3001, 4096, 4097, 5120, 8191, 8192):
+        x = squares_case(kind, n)
+        w = O.normal(n + 2, n, 1.0, 0.1)
+        got, want = H.rms_norm(ctx, x, w, 1e-6), O.rms_norm(x, w, 1e-6)
+        assert (np.isnan(got) == np.isnan(want)).all(), n
+        ok = ~np.isnan(want)
+        assert same_bits(got[ok], want[ok]), n
+
+
 def test_residual_rms_norm_rows_on_device(ctx):
     rows, n = 5, 2048
     x = O.normal(31, rows * n)
