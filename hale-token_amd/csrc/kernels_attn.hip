@@ -434,162 +434,196 @@ __global__ __launch_bounds__(256) void k_attn_ctx(const float* __restrict__ prob
   }
 }
 
-// softmax_in_place and the context in one kernel for score rows up to
-// SMC_MAX positions: work-group (key/value head, 16 columns, 2 query heads)
-// as in k_attn_ctx.  It reads its heads' scores into LDS, takes each head's
-// max, then lanes 0 and 1 of wave 0 carry the two heads' in-order sums of
-// the exp values while waves 1-3 form the exponentials SM_PIPE positions
-// ahead.  The context follows as in k_attn_ctx, except that a product's
-// probability is formed where it is used (exp value / sum, the reference's
-// division), and the first value tiles are loaded before the softmax
-// starts.  The eight work-groups of a head pair each repeat its softmax;
-// that work hides under the sum chain, and no probability goes back to
-// memory.
-constexpr int SMC_MAX = 8192;
+// softmax_in_place and the context in one kernel, for score rows up to
+// SMC_MAX positions: a work-group takes one query head and SMC_COLS of its
+// columns.  All waves form the head's exp values in LDS, four of them sum
+// those in order (ordered_sum.h: K consecutive values per lane), and all
+// divide; then wave 0's lanes carry the context chains, one column each,
+// while waves 1-7 form the products p_t v_t[c] two tiles ahead.
+//
+// Bound by the context chains: one dependent add (2.6 ns) and a quarter of a
+// 16-byte LDS read per position.  The order below takes 3.2 ns: batches of
+// 32 positions with one wait each, the next batch's reads in pairs of
+// additions early in the batch (a read and a wait before every four
+// additions: 3.7 ns), running on over tile borders (a tile's products are
+// complete one barrier before its first read, so the reads need not start
+// anew: 1.2 us per 256 positions otherwise).  The sum was a second such
+// chain before them (4.1 ns per position).  32 heads of 128 over four
+// key/value heads, mean of the lengths up to 3000: 23.4 us with two chains
+// (16 columns of two heads per work-group), 13.7 us so; up to 190: 7.0 and
+// 5.7 us.  32 columns of one head: each work-group forms half as many exp
+// values, and a value row is one 128-byte line.  A head's work-groups repeat
+// its softmax, which no launch boundary then separates from the products.
+// The heads of a group read the same value lines, so grid x is the key/value
+// head and its columns: a multiple of 8 of them keeps a line on one XCD.
+constexpr int SMC_MAX = ORDERED_MAX;
+constexpr int SMC_COLS = 32;
+constexpr int SMC_THREADS = 512;
+constexpr int SMC_T = 128;         // positions per tile, a multiple of 64
+constexpr int SMC_RP = SMC_T + 4;  // row pitch of a product tile: rows 4 banks apart
+constexpr int SMC_LOADERS = SMC_THREADS - 64;  // product threads: waves 1-7
+constexpr int SMC_ITEMS = (SMC_T * SMC_COLS / 4 + SMC_LOADERS - 1) / SMC_LOADERS;  // per product thread
+// exp values in LDS: 4 floats of padding every 32, as in k_rms_norm
+__device__ __host__ constexpr int exp_at(int t) { return t + (t >> 5) * 4; }
 
-__global__ __launch_bounds__(256) void k_attn_softmax_ctx(const float* __restrict__ scores,
-                                                          const float* __restrict__ values, int hd,
-                                                          int kv_dim, int group, int seq, int ld,
-                                                          float* __restrict__ ctx) {
-  constexpr int T = CTX_T, RP = CTX_RP;
-  __shared__ __attribute__((aligned(16))) float ebuf[CTX_HEADS][SMC_MAX];
-  __shared__ __attribute__((aligned(16))) float prod[2][CTX_HEADS * CTX_COLS * RP];
-  __shared__ float red[CTX_HEADS][4];
-  __shared__ float s_sum[CTX_HEADS];
-  const int g = blockIdx.x;               // key/value head
-  const int c0 = blockIdx.y * CTX_COLS;   // first column
-  const int h0 = blockIdx.z * CTX_HEADS;  // first query head within the group
-  const int nh = min(CTX_HEADS, group - h0);
+template <int K>  // 256 K >= seq
+__global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(const float* __restrict__ scores,
+                                                                  const float* __restrict__ values, int hd,
+                                                                  int kv_dim, int group, int seq, int ld,
+                                                                  float* __restrict__ ctx) {
+  constexpr int T = SMC_T, RP = SMC_RP, NBUF = 3;
+  __shared__ __attribute__((aligned(16))) float ebuf[exp_at(256 * K)];
+  __shared__ __attribute__((aligned(16))) float prod[NBUF][SMC_COLS * RP];
+  __shared__ float red[SMC_THREADS / 64];
+  __shared__ float part[ordered_lds(4)];
+  const int blocks = (hd + SMC_COLS - 1) / SMC_COLS;  // column blocks of a head
+  const int g = blockIdx.x / blocks;                  // key/value head
+  const int c0 = blockIdx.x % blocks * SMC_COLS;      // first column
+  const int ncols = min(SMC_COLS, hd - c0);           // a multiple of 16
+  const int h = g * group + blockIdx.y;               // query head
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ntiles = (seq + T - 1) / T;
-  auto tile_n = [&](int ti) { return min(T, seq - ti * T); };
-  const float* srow = scores + ((size_t)g * group + h0) * ld;
+  const float* srow = scores + (size_t)h * ld;
 
-  // value items of waves 1-3 (as in k_attn_ctx); the first NST tiles go out
-  // before the softmax
-  constexpr int NLOAD = 192;
-  const int lt = tid - 64;
+  // value items of the product threads: item i of a tile is position i / 8, columns
+  // 4q .. 4q + 3 with q = i % 8; the first NST tiles go out before the softmax
+  // (every load unconditional, clamped to the last position and column: under
+  // a branch each one would wait for the load before it)
+  constexpr int NLOAD = SMC_LOADERS;
+  const int lt = max(tid - 64, 0);  // wave 0 repeats the first item's loads
   const float* vbase = values + (size_t)g * hd + c0;
   constexpr int NST = 4;
-  f32x4 r[NST][CTX_ITEMS];
+  f32x4 r[NST][SMC_ITEMS];
   auto load = [&](f32x4* R, int ti) {
-    if (ti >= ntiles || lt < 0) return;
-    const int t0 = ti * T, n = tile_n(ti);
-    const float* vb = vbase + (size_t)t0 * kv_dim;
 #pragma unroll
-    for (int j = 0; j < CTX_ITEMS; j++) {
-      const int i = lt + NLOAD * j, t = i / 4, q = i % 4;
-      if (i < T * 4 && t < n) R[j] = *(const f32x4*)(vb + (size_t)t * kv_dim + 4 * q);
+    for (int j = 0; j < SMC_ITEMS; j++) {
+      const int i = lt + NLOAD * j, t = min(ti * T + i / 8, seq - 1), c = min(4 * (i % 8), ncols - 4);
+      R[j] = *(const f32x4*)(vbase + (size_t)t * kv_dim + c);
     }
   };
+  // the head's scores, then its values: loads return in order
+  constexpr int SPT = (256 * K + SMC_THREADS - 1) / SMC_THREADS;
+  float sc[SPT];
+#pragma unroll
+  for (int j = 0; j < SPT; j++) {
+    const int t = tid + SMC_THREADS * j;
+    sc[j] = t < seq ? srow[t] : -INFINITY;
+  }
 #pragma unroll
   for (int j = 0; j < NST; j++) load(r[j], j);
 
-  // softmax: each head's max (order-free; both heads' loads in flight
-  // together), exp values in place, in-order sum
-  float mx[CTX_HEADS];
-  {
-    float m[CTX_HEADS];
+  // max: fold(-inf, f32::max); order-free (a NaN is skipped either way)
+  float m = -INFINITY;
 #pragma unroll
-    for (int hh = 0; hh < CTX_HEADS; hh++) m[hh] = -INFINITY;
-    for (int t0 = tid; t0 < seq; t0 += 256 * 16) {
-      float v[CTX_HEADS][16];
+  for (int j = 0; j < SPT; j++) m = fmaxf(m, sc[j]);
+  m = wave_max_f32(m);
+  if (lane == 0) red[wave] = m;
+  ExpTable tab;
+  tab.load();
+  __syncthreads();
+  m = red[0];
 #pragma unroll
-      for (int hh = 0; hh < CTX_HEADS; hh++)
+  for (int i = 1; i < SMC_THREADS / 64; i++) m = fmaxf(m, red[i]);
 #pragma unroll
-        for (int j = 0; j < 16; j++) {
-          const int t = t0 + 256 * j;
-          v[hh][j] = hh < nh && t < seq ? srow[(size_t)hh * ld + t] : -INFINITY;
-        }
-#pragma unroll
-      for (int hh = 0; hh < CTX_HEADS; hh++)
-#pragma unroll
-        for (int j = 0; j < 16; j++) {
-          const int t = t0 + 256 * j;
-          m[hh] = fmaxf(m[hh], v[hh][j]);
-          if (hh < nh && t < seq) ebuf[hh][t] = v[hh][j];
-        }
-    }
-#pragma unroll
-    for (int hh = 0; hh < CTX_HEADS; hh++) {
-      const float mw = wave_max_f32(m[hh]);
-      if (lane == 0) red[hh][wave] = mw;
-    }
+  for (int j = 0; j < SPT; j++) {
+    const int t = tid + SMC_THREADS * j;
+    sc[j] = wave_expf(sc[j] - m, tab);  // every lane takes part
+    if (t >= seq) sc[j] = 0.0f;
+    if (t < 256 * K) ebuf[exp_at(t)] = sc[j];
   }
   __syncthreads();
+  float v[K];
 #pragma unroll
-  for (int hh = 0; hh < CTX_HEADS; hh++)
-    mx[hh] = fmaxf(fmaxf(red[hh][0], red[hh][1]), fmaxf(red[hh][2], red[hh][3]));
-  // blocks of the sum: a short first block (the chains start sooner), then
-  // SM_PIPE positions each
-  constexpr int FIRST = 128;
-  auto bstart = [&](int k) { return k == 0 ? 0 : min(seq, FIRST + (k - 1) * SM_PIPE); };
-  const int nblk = 1 + (max(0, seq - FIRST) + SM_PIPE - 1) / SM_PIPE;
-  auto expo = [&](int k) {  // waves 1-3: the exp values of block k of every head
-    const int b0 = bstart(k), len = bstart(k + 1) - b0;
-    for (int i = lt; i < nh * len; i += NLOAD) {
-      const int hh = i / len, t = b0 + i % len;
-      ebuf[hh][t] = hale_expf(ebuf[hh][t] - (hh ? mx[1] : mx[0]));
-    }
-  };
-  float sum = 0.0f;  // lane hh of wave 0: sum += exp(v - max), index order
-  if (lt >= 0) expo(0);
-  __syncthreads();
-  for (int k = 0; k < nblk; k++) {
-    if (wave == 0) {
-      if (lane < nh) sum = lds_sum_in_order_a16(&ebuf[lane][bstart(k)], bstart(k + 1) - bstart(k), sum);
-    } else if (k + 1 < nblk) {
-      expo(k + 1);
-    }
-    __syncthreads();
+  for (int k = 0; k < K; k++) v[k] = ebuf[exp_at((tid & 255) * K + k)];
+  const float sum = team_sum_in_order<K>(v, 0.0f, wave, (seq + 64 * K - 1) / (64 * K), part);
+#pragma unroll
+  for (int j = 0; j < SPT; j++) {
+    const int t = tid + SMC_THREADS * j;
+    if (t < seq) ebuf[exp_at(t)] = sc[j] / sum;
   }
-  if (wave == 0 && lane < nh) s_sum[lane] = sum;
   __syncthreads();
-  float sm[CTX_HEADS];
-#pragma unroll
-  for (int hh = 0; hh < CTX_HEADS; hh++) sm[hh] = hh < nh ? s_sum[hh] : 1.0f;
 
-  // context: products p_t v_t[c] with p_t = e_t / sum, tile i + 1 formed
-  // while the chains add tile i
-  auto multiply = [&](const f32x4* R, int ti, int b) {
-    if (lt < 0) return;
-    const int t0 = ti * T, n = tile_n(ti);
+  if (wave == 0) {
+    // two barriers before the first tile (tiles 0 and 1 are formed), then
+    // one per tile.  Positions past the end carry +0 products: acc starts at
+    // +0 and so is never the -0 that they would change.
+    const f32x4* col = (const f32x4*)&prod[0][(lane & (SMC_COLS - 1)) * RP];  // lanes 32-63 repeat
+    constexpr int BUF = SMC_COLS * RP / 4;
+    f32x4 A[8], B[8];
+    float acc = 0.0f;
+    auto batch = [&](const f32x4* X, f32x4* Y, const f32x4* next) {
+      asm volatile("" ::"v"(X[7].w));  // the batch's one wait
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < CTX_ITEMS; j++) {
-      const int i = lt + NLOAD * j, t = i / 4, q = i % 4;
-      if (i < T * 4 && t < n) {
+      for (int q = 0; q < 8; q++) {
+        if (q < 4) Y[2 * q] = next[2 * q];
+        __builtin_amdgcn_sched_barrier(0);
+        acc = acc + X[q].x;
+        acc = acc + X[q].y;
+        __builtin_amdgcn_sched_barrier(0);
+        if (q < 4) Y[2 * q + 1] = next[2 * q + 1];
+        __builtin_amdgcn_sched_barrier(0);
+        acc = acc + X[q].z;
+        acc = acc + X[q].w;
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    __syncthreads();
 #pragma unroll
-        for (int hh = 0; hh < CTX_HEADS; hh++) {
-          if (hh < nh) {
-            const float pr = ebuf[hh][t0 + t] / sm[hh];
-            float* d = &prod[b][(hh * CTX_COLS + 4 * q) * RP + t];
-            d[0] = pr * R[j].x;
-            d[RP] = pr * R[j].y;
-            d[2 * RP] = pr * R[j].z;
-            d[3 * RP] = pr * R[j].w;
-          }
-        }
+    for (int q = 0; q < 8; q++) A[q] = col[q];
+    int buf = 0;
+    __syncthreads();
+    for (int ti = 0; ti < ntiles; ti++) {
+      const f32x4* p = col + buf * BUF;
+      buf = buf + 1 == NBUF ? 0 : buf + 1;
+      const f32x4* after = col + buf * BUF;  // the next tile's first batch (stale after the last tile)
+      const int nb = (min(T, seq - ti * T) + 63) / 64;
+      for (int i = 0; i < nb; i++) {
+        batch(A, B, p + 8);
+        p += 16;
+        batch(B, A, i + 1 < nb ? p : after);
+      }
+      __syncthreads();
+    }
+    if (lane < ncols) ctx[(size_t)h * hd + c0 + lane] = acc;
+    return;
+  }
+  auto multiply = [&](const f32x4* R, int ti) {
+    const int t0 = ti * T, n = min(T, seq - t0), n64 = (n + 63) & ~63;
+    float* P = prod[ti % NBUF];
+#pragma unroll
+    for (int j = 0; j < SMC_ITEMS; j++) {
+      const int i = lt + NLOAD * j, t = i / 8, q = i % 8;
+      const bool in = t < n;
+      const float pr = ebuf[exp_at(min(t0 + t, seq - 1))];
+      if (t < n64 && 4 * q < ncols) {
+        float* d = P + 4 * q * RP + t;
+        d[0] = in ? pr * R[j].x : 0.0f;
+        d[RP] = in ? pr * R[j].y : 0.0f;
+        d[2 * RP] = in ? pr * R[j].z : 0.0f;
+        d[3 * RP] = in ? pr * R[j].w : 0.0f;
       }
     }
   };
-  const bool chain = tid < nh * CTX_COLS;
-  float acc = 0.0f;
-  if (ntiles > 0) multiply(r[0], 0, 0);
+  // stage s holds the tiles ti with ti % NST == s
+  multiply(r[0], 0);
+  load(r[0], NST);
+  __syncthreads();
+  if (ntiles > 1) multiply(r[1], 1);
+  load(r[1], NST + 1);
   __syncthreads();
   for (int ti0 = 0; ti0 < ntiles; ti0 += NST) {
 #pragma unroll
     for (int j = 0; j < NST; j++) {
       const int ti = ti0 + j;  // the chains add tile ti
       if (ti < ntiles) {
-        if (chain) acc = lds_sum_in_order_a16(&prod[ti & 1][tid * RP], tile_n(ti), acc);
-        if (ti + 1 < ntiles) multiply(r[(j + 1) % NST], ti + 1, (ti + 1) & 1);
-        load(r[j], ti + NST);  // its products went to LDS one iteration ago
+        if (ti + 2 < ntiles) multiply(r[(j + 2) % NST], ti + 2);
+        load(r[(j + 2) % NST], ti + 2 + NST);  // its products are formed
         __syncthreads();
       }
     }
   }
-  if (chain) ctx[(size_t)(g * group + h0 + tid / CTX_COLS) * hd + c0 + tid % CTX_COLS] = acc;
 }
 
 hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t rows, size_t n,
@@ -618,13 +652,21 @@ hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {
   const int group = a.nh / a.nkv;
   dim3 gs((unsigned)((a.seq + SC_POS - 1) / SC_POS), (unsigned)a.nkv,
           (unsigned)((group + SC_HEADS - 1) / SC_HEADS));
-  e = launch(k_attn_scores, gs, 256, 0, st, (const float*)a.q, (const float*)a.keys, a.hd, kv_dim,
-             a.nh / a.nkv, a.seq, a.ld, scale, a.scores);
+  e = launch(k_attn_scores, gs, 256, 0, st, (const float*)a.q, (const float*)a.keys, a.hd, kv_dim, group, a.seq, a.ld, scale, a.scores);
   if (e != hipSuccess) return e;
+  if (a.seq <= SMC_MAX) {
+    const dim3 grid((unsigned)(a.nkv * ((a.hd + SMC_COLS - 1) / SMC_COLS)), (unsigned)group);
+    auto run = [&](auto kernel) {
+      return launch(kernel, grid, SMC_THREADS, 0, st, (const float*)a.scores, (const float*)a.values, a.hd, kv_dim,
+                    group, a.seq, a.ld, a.ctx);
+    };
+    if (a.seq <= 512) return run(k_attn_softmax_ctx<2>);
+    if (a.seq <= 1024) return run(k_attn_softmax_ctx<4>);
+    if (a.seq <= 2048) return run(k_attn_softmax_ctx<8>);
+    if (a.seq <= 4096) return run(k_attn_softmax_ctx<16>);
+    return run(k_attn_softmax_ctx<32>);
+  }
   dim3 gc((unsigned)a.nkv, (unsigned)(a.hd / CTX_COLS), (unsigned)((group + CTX_HEADS - 1) / CTX_HEADS));
-  if (a.seq <= SMC_MAX)
-    return launch(k_attn_softmax_ctx, gc, 256, 0, st, (const float*)a.scores,
-                  (const float*)a.values, a.hd, kv_dim, group, a.seq, a.ld, a.ctx);
   e = launch(k_attn_softmax, (unsigned)a.nh, 256, 0, st, a.scores, a.seq, a.ld);
   if (e != hipSuccess) return e;
   return launch(k_attn_ctx, gc, 256, 0, st, (const float*)a.scores,

@@ -49,8 +49,7 @@ __device__ __forceinline__ float dpp_up(float id, float x) {
 // wave w holding the K values from (64 w + l) K on (0 past the end, at most
 // ORDERED_MAX in all, each >= +0, infinite or NaN).  acc >= +0 is the sum so
 // far.  Every thread of the work-group calls it together (it synchronizes
-// 1 + nw times; a work-group may hold several teams of nw waves, each with
-// its own `lds`); every thread of a team gets the sum.
+// 1 + nw times); waves from nw on add nothing, and every thread gets the sum.
 template <int K>
 __device__ __forceinline__ float team_sum_in_order(const float (&v)[K], float acc, int w, int nw,
                                                    float* lds) {
@@ -72,13 +71,13 @@ __device__ __forceinline__ float team_sum_in_order(const float (&v)[K], float ac
   top = fmaxf(top, dpp_up<C, R>(0.0f, top));
   HALE_SCAN_STEPS(HALE_STEP)
 #undef HALE_STEP
-  if (__lane_id() == 63) {
+  if (w < nw && __lane_id() == 63) {
     lds[w] = incl;
     lds[nw + w] = top;
   }
   __syncthreads();
   float base = acc, floor_ = acc;
-  for (int i = 0; i < w; i++) {
+  for (int i = 0; i < min(w, nw); i++) {
     base = base + lds[i];
     floor_ = fmaxf(floor_, lds[nw + i]);
   }

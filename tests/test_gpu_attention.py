@@ -158,6 +158,23 @@ def test_attention_long_context(ctx, nh, nkv, hd):
     att.close()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,steps", [(2, 1, 80, 2060), (3, 1, 48, 520), (2, 2, 16, 4100)])
+def test_attention_softmax_context_edges(ctx, nh, nkv, hd, steps):
+    # both sides of the row lengths that pick the values per lane of the
+    # ordered sum, of the 128-position tiles and of their 64-position batches,
+    # with head sizes whose last column block is half full
+    ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=hd, qk_norm=True, max_len=steps)
+    edges = {n - 1 for c in (1, 32, 64, 128, 192, 256, 384, 512, 1024, 2048, 4096) for n in (c, c + 1, c + 2)}
+    for pos in range(steps):
+        x = O.normal(9000 + pos, 64, 0.0, 3.0)
+        c, s = O.rope_angles(hd, 1e6, pos)
+        got = att.forward(x, pos, c, s)
+        want = ref.forward(x, c, s)
+        if pos in edges or pos == steps - 1:
+            assert same_bits(got, want), pos
+    att.close()
+
+
 def test_attention_softmax_past_one_lds_chunk(ctx):
     # rows up to 8192 positions run softmax and context in one kernel, longer
     # ones in two; a score row longer than the softmax keeps in LDS (12288)
