@@ -228,11 +228,12 @@ hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t 
                            float eps, float* out, hipStream_t st);
 
 // One token of grouped-query attention after the q/k/v projections: QK-norm
-// and RoPE of q and k, k/v pushed to the cache at row seq - 1, scores,
-// softmax and the context.  keys/values are [ld][nkv*hd] f32, scores
+// and RoPE of q and k, k/v pushed to the cache at position seq - 1, scores,
+// softmax and the context.  keys and values hold cap * nkv * hd f32 each,
+// values as [cap][nkv*hd], keys as kernels_attn.hip lays them out; scores
 // [nh][ld], ctx [nh*hd].
 struct AttnArgs {
-  float* q;            // [nh*hd], normalised and rotated in place
+  const float* q;      // [nh*hd] projection output
   const float* k;      // [nkv*hd] projection output
   const float* v;      // [nkv*hd]
   int nh, nkv, hd;
@@ -244,7 +245,8 @@ struct AttnArgs {
   float* keys;
   float* values;
   int seq;              // positions after the push (position + 1)
-  int ld;               // cache capacity (rows of keys/values, row stride of scores)
+  int cap;              // cache capacity (positions)
+  int ld;               // row stride of scores
   float* scores;
   float* ctx;
 };

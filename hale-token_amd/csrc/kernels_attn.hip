@@ -24,18 +24,6 @@ namespace hale {
 constexpr int NORM_MAX = ORDERED_MAX;  // elements of an RMSNorm row
 constexpr int HEAD_MAX = 1024;     // largest head_dim
 
-// inverse_rms (src/ops/norm.rs:25-28) of n values whose squares are in
-// sq[0, n) of LDS; every thread gets the scale.  One chain: for a head's
-// 64-128 values the lanes' scan (ordered_sum.h) would take as long.
-__device__ __forceinline__ float block_inverse_rms(const float* sq, int n, float eps, float* bcast) {
-  if (threadIdx.x == 0) {
-    const float s = lds_sum_in_order(sq, n, -0.0f);
-    bcast[0] = 1.0f / sqrtf(s / (float)n + eps);
-  }
-  __syncthreads();
-  return bcast[0];
-}
-
 // One work-group per row: out = rms_norm(x + delta, w) with x updated to
 // x + delta first when delta is given (add_in_place, then rms_norm).  The
 // row and the weights are read once, all loads in flight together, and stay
@@ -113,121 +101,253 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
   }
 }
 
-// QK-norm and RoPE of every query and key head, then the cache push.
-// Work-group h < nh: query head h (in place in q).  nh <= h < nh + nkv: key
-// head h - nh, written to keys[pos]; the same work-group copies value head
-// h - nh to values[pos].
-__global__ __launch_bounds__(64) void k_qk_norm_rope(float* __restrict__ q, const float* __restrict__ k,
-                                                     const float* __restrict__ v, int nh, int hd,
-                                                     const float* __restrict__ q_norm,
-                                                     const float* __restrict__ k_norm, float eps,
-                                                     const float* __restrict__ cos,
-                                                     const float* __restrict__ sin,
-                                                     float* __restrict__ keys_pos,
-                                                     float* __restrict__ values_pos) {
-  __shared__ __attribute__((aligned(16))) float head[HEAD_MAX];
-  __shared__ __attribute__((aligned(16))) float sq[HEAD_MAX];
-  __shared__ float bcast[1];
-  const int hb = blockIdx.x;
-  const bool is_q = hb < nh;
-  const int h = is_q ? hb : hb - nh;
-  const float* src = is_q ? q + (size_t)h * hd : k + (size_t)h * hd;
-  float* dst = is_q ? q + (size_t)h * hd : keys_pos + (size_t)h * hd;
-  const float* wn = is_q ? q_norm : k_norm;
-  for (int i = threadIdx.x; i < hd; i += 64) {
-    const float a = src[i];
-    head[i] = a;
-    sq[i] = a * a;
+// One token's projections and what becomes of them (AttnArgs without the
+// buffers between the kernels).
+struct TokenArgs {
+  const float *q, *k, *v;         // projection outputs
+  const float *q_norm, *k_norm;   // [hd] or null
+  const float *cos, *sin;         // [hd / 2]
+  float eps;
+  float *keys, *values;           // the layer cache
+  int hd, kv_dim, group, cap, seq;
+};
+
+// The cache: values [position][nkv * hd]; keys head by head in pieces of four
+// dimensions, [head][hd / 4][position][4], so that a wave whose lanes take one
+// position each reads a piece of 64 positions as one kilobyte.
+__device__ __forceinline__ size_t key_piece(const TokenArgs& a, int g, int piece, int t) {
+  return (((size_t)g * (a.hd / 4) + piece) * a.cap + t) * 4;
+}
+
+// Orders a wave's LDS accesses: what its lanes wrote, any of them now reads.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// QK-norm and RoPE of R heads by one wave, into LDS rows of hd + 4 floats (the
+// padding keeps the rows' 16-byte reads 4 banks apart).  load() takes the
+// first 128 values of each head and what they are multiplied with into
+// registers, unconditionally, so that the key loads which follow it can stay
+// in flight while store() runs: loads return in order.  The norm's sum of hd
+// squares is one chain per head, a lane each (0.5 us for 128 values).
+template <int R>
+struct HeadRows {
+  const float* src[R];   // wave-uniform
+  const float* norm[R];  // or null
+  float x[R][2], w[R][2], cs, sn;
+  __device__ __forceinline__ void load(const TokenArgs& a) {
+    const int lane = __lane_id(), last = a.hd - 1, half = a.hd / 2;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+#pragma unroll
+      for (int j = 0; j < 2; j++) {
+        x[r][j] = src[r][min(lane + 64 * j, last)];
+        w[r][j] = (norm[r] ? norm[r] : src[r])[min(lane + 64 * j, last)];
+      }
+    cs = a.cos[min(lane, half - 1)];
+    sn = a.sin[min(lane, half - 1)];
   }
-  if (!is_q)
-    for (int i = threadIdx.x; i < hd; i += 64) values_pos[(size_t)h * hd + i] = v[(size_t)h * hd + i];
-  __syncthreads();
-  if (wn) {  // rms_norm_in_place: x = x * (scale * w)
-    const float scale = block_inverse_rms(sq, hd, eps, bcast);
-    for (int i = threadIdx.x; i < hd; i += 64) head[i] = head[i] * (scale * wn[i]);
-    __syncthreads();
+  __device__ __forceinline__ void store(const TokenArgs& a, float* rows) {
+    const int lane = __lane_id(), hd = a.hd, half = hd / 2, pitch = hd + 4;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        if (lane + 64 * j < hd) rows[r * pitch + lane + 64 * j] = x[r][j];
+      for (int c = 128 + lane; c < hd; c += 64) rows[r * pitch + c] = src[r][c];
+    }
+    wave_lds_sync();
+    float scale = 0.0f;  // inverse_rms (src/ops/norm.rs:25-28), in order from -0.0
+    if (lane < R) {
+      const f32x4* row = (const f32x4*)(rows + lane * pitch);
+      float s = -0.0f;
+#pragma unroll 8
+      for (int i = 0; i < hd / 4; i++) {
+        const f32x4 v = row[i];
+        s = s + v.x * v.x;
+        s = s + v.y * v.y;
+        s = s + v.z * v.z;
+        s = s + v.w * v.w;
+      }
+      scale = 1.0f / sqrtf(s / (float)hd + a.eps);
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const float sc = lane_value(scale, r);
+      const bool normed = norm[r] != nullptr;
+      float* row = rows + r * pitch;
+      // rms_norm_in_place: x = x * (scale * w)
+      if (hd <= 128) {
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+          if (lane + 64 * j < hd) row[lane + 64 * j] = normed ? x[r][j] * (sc * w[r][j]) : x[r][j];
+      } else if (normed) {
+        for (int c = lane; c < hd; c += 64) row[c] = row[c] * (sc * norm[r][c]);
+      }
+      wave_lds_sync();
+      for (int c = lane; c < half; c += 64) {  // Rope::apply (src/ops/rope.rs:36-44)
+        const float p = row[c], q = row[half + c];
+        const float cc = c < 64 ? cs : a.cos[c], ss = c < 64 ? sn : a.sin[c];
+        row[c] = p * cc - q * ss;
+        row[half + c] = q * cc + p * ss;
+      }
+    }
+    wave_lds_sync();
   }
-  const int half = hd / 2;  // Rope::apply (src/ops/rope.rs:36-44)
-  for (int i = threadIdx.x; i < half; i += 64) {
-    const float a = head[i], b = head[half + i];
-    dst[i] = a * cos[i] - b * sin[i];
-    dst[half + i] = b * cos[i] + a * sin[i];
+};
+
+// LayerCache::push of key/value head g (src/model/kv_cache.rs): the prepared
+// key row and the value projection, by one wave.
+__device__ __forceinline__ void push_head(const TokenArgs& a, int g, const float* krow) {
+  for (int i = __lane_id(); i < a.hd; i += 64) {
+    a.keys[key_piece(a, g, i / 4, a.seq - 1) + i % 4] = krow[i];
+    a.values[(size_t)(a.seq - 1) * a.kv_dim + (size_t)g * a.hd + i] = a.v[(size_t)g * a.hd + i];
   }
 }
 
-// scores[h][t] = (q_h . key_t) * scale for t < seq: the dot product in
-// index order from -0.0 (Iterator::sum), then one multiply.  A work-group
-// takes SC_POS positions of one key/value head for up to SC_HEADS query
-// heads of its group (thread (query head, position) carries one chain), so
-// every key row is read once per group.  Keys and the queries stream
-// through LDS in chunks of SC_W dimensions: coalesced 16-byte loads (four
-// lanes per 64-byte row piece), chunk c + 1 in registers while chunk c is
-// added, and each chain reads its 4 key and 4 query values per 16-byte read.
-constexpr int SC_POS = 32;
-constexpr int SC_HEADS = 8;
-constexpr int SC_W = 16;
-constexpr int SC_KP = SC_W + 4;  // key row pitch in LDS
+// q . k in index order from -0.0 (Iterator::sum) of one query row and one
+// key row in LDS.
+__device__ __forceinline__ float dot_rows(const float* q, const float* k, int hd) {
+  const f32x4 *q4 = (const f32x4*)q, *k4 = (const f32x4*)k;
+  float s = -0.0f;
+#pragma unroll 8
+  for (int i = 0; i < hd / 4; i++) {
+    const f32x4 x = q4[i], y = k4[i];
+    s = s + x.x * y.x;
+    s = s + x.y * y.y;
+    s = s + x.z * y.z;
+    s = s + x.w * y.w;
+  }
+  return s;
+}
 
-__global__ __launch_bounds__(256) void k_attn_scores(const float* __restrict__ q,
-                                                     const float* __restrict__ keys, int hd,
-                                                     int kv_dim, int group, int seq, int ld,
-                                                     float scale, float* __restrict__ scores) {
-  __shared__ __attribute__((aligned(16))) float kt[2][SC_POS * SC_KP];
-  __shared__ __attribute__((aligned(16))) float qt[2][SC_HEADS * SC_W];
-  const int g = blockIdx.y;                // key/value head
-  const int h0 = blockIdx.z * SC_HEADS;    // first query head within the group
-  const int nhq = min(SC_HEADS, group - h0);
-  // work-group x runs on XCD x % 8: give each XCD a contiguous run of
-  // position blocks, so each score row is written in long runs per XCD
-  const int nbx = gridDim.x;
-  const int bx = nbx % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nbx / 8) + (int)blockIdx.x / 8;
-  const int t0 = bx * SC_POS;
-  const int tid = threadIdx.x;
-  const int hq = tid / SC_POS, tp = tid % SC_POS;
-  const bool chain = hq < nhq && t0 + tp < seq;
-  const int nc = hd / SC_W;
-  // loads of one chunk: threads 0-127 a float4 of the keys (row tid / 4,
-  // part tid % 4), threads 128 .. 128 + 4 nhq a float4 of the queries
-  const int kr = tid / 4, kq = tid % 4;
-  const bool kload = tid < SC_POS * 4 && t0 + kr < seq;
-  const int qi = tid - SC_POS * 4, qh = qi / 4, qq = qi % 4;
-  const bool qload = qi >= 0 && qh < nhq;
-  const float* krow = keys + (size_t)(t0 + kr) * kv_dim + g * hd + 4 * kq;
-  const float* qrow = q + (size_t)(g * group + h0 + qh) * hd + 4 * qq;
-  f32x4 reg = {};
-  auto load = [&](int c) {
-    if (kload) reg = *(const f32x4*)(krow + SC_W * c);
-    if (qload) reg = *(const f32x4*)(qrow + SC_W * c);
-  };
-  auto store = [&](int b) {
-    if (kload) *(f32x4*)&kt[b][kr * SC_KP + 4 * kq] = reg;
-    if (qload) *(f32x4*)&qt[b][qh * SC_W + 4 * qq] = reg;
-  };
-  float s = -0.0f;  // Iterator::sum
-  load(0);
-  store(0);
-  if (nc > 1) load(1);
-  __syncthreads();
-  for (int c = 0; c < nc; c++) {
-    if (chain) {
-      const f32x4* kk = (const f32x4*)&kt[c & 1][tp * SC_KP];
-      const f32x4* qv = (const f32x4*)&qt[c & 1][hq * SC_W];
+// The same for the cached key rows of the lanes' positions (clamped by the
+// caller) against NQ query rows in LDS, pieces of KEY_CHUNK dimensions in
+// two register sets: start() sends the first two for before the query rows
+// exist, so that a head of 128 has one round trip.
+constexpr int KEY_CHUNK = 64;
+template <int NQ>
+struct KeyDots {
+  f32x4 r[2][KEY_CHUNK / 4];
+  const float* base;
+  size_t step;  // floats from a piece to the next
+  int pieces;
+  __device__ __forceinline__ void load(f32x4* d, int chunk) {
 #pragma unroll
-      for (int u = 0; u < SC_W / 4; u++) {
-        const f32x4 a = qv[u], b = kk[u];
-        s = s + a.x * b.x;
-        s = s + a.y * b.y;
-        s = s + a.z * b.z;
-        s = s + a.w * b.w;
+    for (int i = 0; i < KEY_CHUNK / 4; i++)
+      d[i] = *(const f32x4*)(base + (size_t)min(chunk * (KEY_CHUNK / 4) + i, pieces - 1) * step);
+  }
+  __device__ __forceinline__ void start(const TokenArgs& a, int g, int t) {
+    base = a.keys + key_piece(a, g, 0, t);
+    step = (size_t)a.cap * 4;
+    pieces = a.hd / 4;
+    load(r[0], 0);
+    load(r[1], 1);
+  }
+  __device__ __forceinline__ void add(const f32x4* d, int chunk, const float* q, int pitch, float* s) {
+#pragma unroll
+    for (int j = 0; j < KEY_CHUNK / 16; j++) {
+      const int p0 = chunk * (KEY_CHUNK / 4) + 4 * j;
+      if (p0 < pieces) {  // uniform; hd is a multiple of 16
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const f32x4 y = d[4 * j + i];
+#pragma unroll
+          for (int h = 0; h < NQ; h++) {
+            const f32x4 x = *(const f32x4*)(q + h * pitch + 4 * (p0 + i));
+            s[h] = s[h] + x.x * y.x;
+            s[h] = s[h] + x.y * y.y;
+            s[h] = s[h] + x.z * y.z;
+            s[h] = s[h] + x.w * y.w;
+          }
+        }
       }
     }
-    if (c + 1 < nc) {
-      store((c + 1) & 1);  // that buffer was last read in iteration c - 1
-      if (c + 2 < nc) load(c + 2);
-    }
-    __syncthreads();
   }
-  if (chain) scores[(size_t)(g * group + h0 + hq) * ld + t0 + tp] = s * scale;
+  __device__ __forceinline__ void finish(const float* q, int pitch, float* s) {
+#pragma unroll
+    for (int h = 0; h < NQ; h++) s[h] = -0.0f;
+    const int chunks = (pieces + KEY_CHUNK / 4 - 1) / (KEY_CHUNK / 4);
+    for (int c = 0; c < chunks; c += 2) {
+      add(r[0], c, q, pitch, s);
+      if (c + 2 < chunks) load(r[0], c + 2);
+      if (c + 1 < chunks) add(r[1], c + 1, q, pitch, s);
+      if (c + 3 < chunks) load(r[1], c + 3);
+    }
+  }
+};
+
+// scores[h][t] = (q_h . key_t) / sqrt(hd) for t < seq.  A work-group takes 64
+// positions of one key/value head for up to SC_HEADS query heads of its
+// group: lanes are positions, each wave carries SC_WAVE_HEADS heads' chains
+// side by side and norms and rotates those heads itself, under its key loads:
+// 7.6 us (512 - 3000 positions of four key/value heads) where a launch for
+// the norm and one for the scores took 3.7 and 5.0.  The last work-group in
+// x does so for the new key too, pushes it and the new value, and scores it.
+//
+// Bound by latency: launch, key round trip, the chains of two rounded
+// operations per dimension.  A wave's keys come through L1, which a
+// second head per wave halves.  Position blocks are contiguous per XCD
+// (work-group x runs on XCD x % 8): each score row is written in long runs
+// per XCD.
+constexpr int SC_POS = 64;
+constexpr int SC_WAVES = 4;
+constexpr int SC_WAVE_HEADS = 2;
+constexpr int SC_HEADS = SC_WAVES * SC_WAVE_HEADS;
+constexpr int SC_ROWS = SC_WAVE_HEADS + 1;  // LDS rows per wave: its heads, the new key
+
+__global__ __launch_bounds__(64 * SC_WAVES) void k_attn_scores(TokenArgs a, int ld, float scale,
+                                                               float* __restrict__ scores) {
+  extern __shared__ __attribute__((aligned(16))) float s_heads[];  // SC_WAVES * SC_ROWS rows of hd + 4
+  const int g = blockIdx.y;  // key/value head
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pitch = a.hd + 4;
+  // the wave's first head and how many it has (none beyond the group)
+  const int first = (int)blockIdx.z * SC_HEADS + wave * SC_WAVE_HEADS;
+  const int nq = min(SC_WAVE_HEADS, a.group - first);
+  if (nq <= 0) return;
+  const int h0 = g * a.group + first;
+  float* rows = s_heads + (size_t)wave * SC_ROWS * pitch;
+  const int nbx = gridDim.x - 1;  // blocks of cached positions
+  if ((int)blockIdx.x == nbx) {
+    HeadRows<SC_ROWS> heads;
+#pragma unroll
+    for (int r = 0; r < SC_WAVE_HEADS; r++) {
+      heads.src[r] = a.q + (size_t)(h0 + min(r, nq - 1)) * a.hd;
+      heads.norm[r] = a.q_norm;
+    }
+    heads.src[SC_WAVE_HEADS] = a.k + (size_t)g * a.hd;
+    heads.norm[SC_WAVE_HEADS] = a.k_norm;
+    heads.load(a);
+    heads.store(a, rows);
+    const float* krow = rows + SC_WAVE_HEADS * pitch;
+    if (first == 0) push_head(a, g, krow);
+    if (lane < nq) scores[(size_t)(h0 + lane) * ld + a.seq - 1] = dot_rows(rows + lane * pitch, krow, a.hd) * scale;
+    return;
+  }
+  const int bx = nbx % 8 ? (int)blockIdx.x : (int)(blockIdx.x % 8) * (nbx / 8) + (int)blockIdx.x / 8;
+  const int t = bx * SC_POS + lane;
+  HeadRows<SC_WAVE_HEADS> heads;
+#pragma unroll
+  for (int r = 0; r < SC_WAVE_HEADS; r++) {
+    heads.src[r] = a.q + (size_t)(h0 + min(r, nq - 1)) * a.hd;
+    heads.norm[r] = a.q_norm;
+  }
+  heads.load(a);
+  __builtin_amdgcn_sched_barrier(0);
+  KeyDots<SC_WAVE_HEADS> dots;
+  dots.start(a, g, min(t, a.seq - 2));
+  __builtin_amdgcn_sched_barrier(0);
+  heads.store(a, rows);
+  float s[SC_WAVE_HEADS];
+  dots.finish(rows, pitch, s);
+#pragma unroll
+  for (int h = 0; h < SC_WAVE_HEADS; h++)
+    if (h < nq && t < a.seq - 1) scores[(size_t)(h0 + h) * ld + t] = s[h] * scale;
 }
 
 // softmax_in_place over each head's scores (one work-group per head): the
@@ -466,25 +586,34 @@ constexpr int SMC_ITEMS = (SMC_T * SMC_COLS / 4 + SMC_LOADERS - 1) / SMC_LOADERS
 // exp values in LDS: 4 floats of padding every 32, as in k_rms_norm
 __device__ __host__ constexpr int exp_at(int t) { return t + (t >> 5) * 4; }
 
-template <int K>  // 256 K >= seq
-__global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(const float* __restrict__ scores,
-                                                                  const float* __restrict__ values, int hd,
-                                                                  int kv_dim, int group, int seq, int ld,
-                                                                  float* __restrict__ ctx) {
+// SHORT (rows of at most SMC_THREADS positions, K = 2): the same work-group
+// prepares its head and the new key and scores the head itself, a position
+// per thread, so that a token's attention is one launch; the keys are then
+// read once per head and column block, 1.7 us of L1 reads for 512 positions
+// where the score launch takes 5.  The new position's key and value come
+// from the projections: the first work-group of a key/value head pushes them
+// to the cache meanwhile.  Rows up to 190 positions: 9.4 us, where the norm,
+// score and softmax launches took 3.7 + 4.8 + 5.7; up to 512: 10.7 against
+// 15.5.
+template <int K, bool SHORT>  // 256 K >= seq
+__global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(TokenArgs a, const float* __restrict__ scores,
+                                                                  int ld, float scale, float* __restrict__ ctx) {
+  static_assert(!SHORT || K == 2, "a position per thread");
   constexpr int T = SMC_T, RP = SMC_RP, NBUF = 3;
   __shared__ __attribute__((aligned(16))) float ebuf[exp_at(256 * K)];
   __shared__ __attribute__((aligned(16))) float prod[NBUF][SMC_COLS * RP];
   __shared__ float red[SMC_THREADS / 64];
   __shared__ float part[ordered_lds(4)];
+  __shared__ __attribute__((aligned(16))) float s_qk[SHORT ? 2 * (HEAD_MAX + 4) : 4];
+  const int hd = a.hd, kv_dim = a.kv_dim, seq = a.seq;
   const int blocks = (hd + SMC_COLS - 1) / SMC_COLS;  // column blocks of a head
   const int g = blockIdx.x / blocks;                  // key/value head
   const int c0 = blockIdx.x % blocks * SMC_COLS;      // first column
   const int ncols = min(SMC_COLS, hd - c0);           // a multiple of 16
-  const int h = g * group + blockIdx.y;               // query head
+  const int h = g * a.group + blockIdx.y;             // query head
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int ntiles = (seq + T - 1) / T;
-  const float* srow = scores + (size_t)h * ld;
 
   // value items of the product threads: item i of a tile is position i / 8, columns
   // 4q .. 4q + 3 with q = i % 8; the first NST tiles go out before the softmax
@@ -492,26 +621,56 @@ __global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(const float* _
   // a branch each one would wait for the load before it)
   constexpr int NLOAD = SMC_LOADERS;
   const int lt = max(tid - 64, 0);  // wave 0 repeats the first item's loads
-  const float* vbase = values + (size_t)g * hd + c0;
+  const float* vbase = a.values + (size_t)g * hd + c0;
+  const float* vnew = a.v + (size_t)g * hd + c0;
   constexpr int NST = 4;
   f32x4 r[NST][SMC_ITEMS];
   auto load = [&](f32x4* R, int ti) {
 #pragma unroll
     for (int j = 0; j < SMC_ITEMS; j++) {
       const int i = lt + NLOAD * j, t = min(ti * T + i / 8, seq - 1), c = min(4 * (i % 8), ncols - 4);
-      R[j] = *(const f32x4*)(vbase + (size_t)t * kv_dim + c);
+      const float* row = SHORT && t == seq - 1 ? vnew : vbase + (size_t)t * kv_dim;
+      R[j] = *(const f32x4*)(row + c);
     }
   };
   // the head's scores, then its values: loads return in order
   constexpr int SPT = (256 * K + SMC_THREADS - 1) / SMC_THREADS;
   float sc[SPT];
+  if constexpr (SHORT) {
+    const int pitch = hd + 4;
+    HeadRows<1> head;  // wave 0: the query head, wave 1: the new key
+    head.src[0] = wave == 1 ? a.k + (size_t)g * hd : a.q + (size_t)h * hd;
+    head.norm[0] = wave == 1 ? a.k_norm : a.q_norm;
+    head.load(a);
+    __builtin_amdgcn_sched_barrier(0);
+    KeyDots<1> dots;
+    dots.start(a, g, max(min(tid, seq - 2), 0));
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < SPT; j++) {
-    const int t = tid + SMC_THREADS * j;
-    sc[j] = t < seq ? srow[t] : -INFINITY;
+    for (int j = 0; j < NST; j++) load(r[j], j);
+    __builtin_amdgcn_sched_barrier(0);
+    if (wave < 2) head.store(a, s_qk + wave * pitch);
+    __syncthreads();
+    if (c0 == 0 && blockIdx.y == 0 && wave == 6) push_head(a, g, s_qk + pitch);
+    sc[0] = 0.0f;
+    if (wave * 64 < seq - 1) dots.finish(s_qk, pitch, sc);
+    // the new position, the row's last: by a lane of the last wave, whose
+    // own positions few rows reach
+    if (tid == SMC_THREADS - 1) red[0] = dot_rows(s_qk, s_qk + pitch, hd);
+    __syncthreads();
+    if (tid == seq - 1) sc[0] = red[0];
+    sc[0] = tid < seq ? sc[0] * scale : -INFINITY;
+    __syncthreads();
+  } else {
+    const float* srow = scores + (size_t)h * ld;
+#pragma unroll
+    for (int j = 0; j < SPT; j++) {
+      const int t = tid + SMC_THREADS * j;
+      sc[j] = t < seq ? srow[t] : -INFINITY;
+    }
+#pragma unroll
+    for (int j = 0; j < NST; j++) load(r[j], j);
   }
-#pragma unroll
-  for (int j = 0; j < NST; j++) load(r[j], j);
 
   // max: fold(-inf, f32::max); order-free (a NaN is skipped either way)
   float m = -INFINITY;
@@ -638,39 +797,34 @@ hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t 
 }
 
 hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {
-  // head_dim a multiple of 16 (context column blocks), GQA group <= 16
-  // (work-groups of group x 16 threads), score rows 16-byte aligned
+  // head_dim a multiple of 16 (context column blocks, key chunks), GQA group
+  // <= 16, score rows 16-byte aligned
   if (a.hd < 16 || a.hd > HEAD_MAX || a.hd % CTX_COLS || a.nh < 1 || a.nkv < 1 || a.nh % a.nkv ||
-      a.nh / a.nkv > 16 || a.seq < 1 || a.seq > a.ld || a.ld % 4)
+      a.nh / a.nkv > 16 || a.seq < 1 || a.seq > a.cap || a.cap > a.ld || a.ld % 4)
     return hipErrorInvalidValue;
-  const int kv_dim = a.nkv * a.hd;
-  hipError_t e = launch(k_qk_norm_rope, (unsigned)(a.nh + a.nkv), 64, 0, st, a.q, a.k, a.v, a.nh, a.hd,
-                        a.q_norm, a.k_norm, a.eps, a.cos, a.sin, a.keys + (size_t)(a.seq - 1) * kv_dim,
-                        a.values + (size_t)(a.seq - 1) * kv_dim);
-  if (e != hipSuccess) return e;
+  const int kv_dim = a.nkv * a.hd, group = a.nh / a.nkv;
   const float scale = 1.0f / sqrtf((float)a.hd);
-  const int group = a.nh / a.nkv;
-  dim3 gs((unsigned)((a.seq + SC_POS - 1) / SC_POS), (unsigned)a.nkv,
-          (unsigned)((group + SC_HEADS - 1) / SC_HEADS));
-  e = launch(k_attn_scores, gs, 256, 0, st, (const float*)a.q, (const float*)a.keys, a.hd, kv_dim, group, a.seq, a.ld, scale, a.scores);
+  const TokenArgs t{a.q, a.k, a.v, a.q_norm, a.k_norm, a.cos, a.sin, a.eps, a.keys, a.values,
+                    a.hd, kv_dim, group, a.cap, a.seq};
+  const dim3 gsc((unsigned)(a.nkv * ((a.hd + SMC_COLS - 1) / SMC_COLS)), (unsigned)group);
+  auto softmax_ctx = [&](auto kernel) {
+    return launch(kernel, gsc, SMC_THREADS, 0, st, t, (const float*)a.scores, a.ld, scale, a.ctx);
+  };
+  if (a.seq <= SMC_THREADS) return softmax_ctx(k_attn_softmax_ctx<2, true>);
+  const dim3 gs((unsigned)((a.seq - 1 + SC_POS - 1) / SC_POS + 1), (unsigned)a.nkv,
+                (unsigned)((group + SC_HEADS - 1) / SC_HEADS));
+  hipError_t e = launch(k_attn_scores, gs, 64 * SC_WAVES, (uint32_t)(SC_WAVES * SC_ROWS * (a.hd + 4) * sizeof(float)), st,
+                        t, a.ld, scale, a.scores);
   if (e != hipSuccess) return e;
-  if (a.seq <= SMC_MAX) {
-    const dim3 grid((unsigned)(a.nkv * ((a.hd + SMC_COLS - 1) / SMC_COLS)), (unsigned)group);
-    auto run = [&](auto kernel) {
-      return launch(kernel, grid, SMC_THREADS, 0, st, (const float*)a.scores, (const float*)a.values, a.hd, kv_dim,
-                    group, a.seq, a.ld, a.ctx);
-    };
-    if (a.seq <= 512) return run(k_attn_softmax_ctx<2>);
-    if (a.seq <= 1024) return run(k_attn_softmax_ctx<4>);
-    if (a.seq <= 2048) return run(k_attn_softmax_ctx<8>);
-    if (a.seq <= 4096) return run(k_attn_softmax_ctx<16>);
-    return run(k_attn_softmax_ctx<32>);
-  }
-  dim3 gc((unsigned)a.nkv, (unsigned)(a.hd / CTX_COLS), (unsigned)((group + CTX_HEADS - 1) / CTX_HEADS));
+  if (a.seq <= 1024) return softmax_ctx(k_attn_softmax_ctx<4, false>);
+  if (a.seq <= 2048) return softmax_ctx(k_attn_softmax_ctx<8, false>);
+  if (a.seq <= 4096) return softmax_ctx(k_attn_softmax_ctx<16, false>);
+  if (a.seq <= SMC_MAX) return softmax_ctx(k_attn_softmax_ctx<32, false>);
   e = launch(k_attn_softmax, (unsigned)a.nh, 256, 0, st, a.scores, a.seq, a.ld);
   if (e != hipSuccess) return e;
-  return launch(k_attn_ctx, gc, 256, 0, st, (const float*)a.scores,
-                (const float*)a.values, a.hd, kv_dim, group, a.seq, a.ld, a.ctx);
+  const dim3 gc((unsigned)a.nkv, (unsigned)(a.hd / CTX_COLS), (unsigned)((group + CTX_HEADS - 1) / CTX_HEADS));
+  return launch(k_attn_ctx, gc, 256, 0, st, (const float*)a.scores, (const float*)a.values, a.hd, kv_dim, group, a.seq,
+                a.ld, a.ctx);
 }
 
 }  // namespace hale

@@ -2220,7 +2220,7 @@ struct hale_attention {
   size_t H = 0, nh = 0, nkv = 0, hd = 0, max_len = 0, len = 0;
   float eps = 0.0f;
   float *q_norm = nullptr, *k_norm = nullptr;  // [hd] device copies, or null
-  float *keys = nullptr, *values = nullptr;    // the layer cache, [max_len][nkv*hd]
+  float *keys = nullptr, *values = nullptr;    // the layer cache, max_len positions
   // per-call buffers: q, k, v, context, scores [nh][max_len], x/cos/sin/out
   // staging of the host entry point, q8 activation blocks
   float *dq = nullptr, *dk = nullptr, *dv = nullptr, *dctx = nullptr, *scores = nullptr;
@@ -2286,7 +2286,7 @@ extern "C" int hale_attention_create(hale_ctx* c, const hale_matrix* q, const ha
   ALLOC(a->dk, kv_dim * 4);
   ALLOC(a->dv, kv_dim * 4);
   ALLOC(a->dctx, nh * hd * 4);
-  ALLOC(a->scores, nh * ((max_len + 3) / 4 * 4) * 4);
+  ALLOC(a->scores, nh * ((max_len + 31) / 32 * 32) * 4);
   ALLOC(a->hx, H * 4);
   ALLOC(a->hcos, hd * 2);
   ALLOC(a->hsin, hd * 2);
@@ -2347,7 +2347,8 @@ extern "C" int hale_attention_forward_device(hale_attention* a, const float* d_x
   t.keys = a->keys;
   t.values = a->values;
   t.seq = (int)position + 1;
-  t.ld = (int)((a->max_len + 3) / 4 * 4);  // score rows 16-byte aligned
+  t.cap = (int)a->max_len;
+  t.ld = (int)((a->max_len + 31) / 32 * 32);  // score rows of whole 128-byte lines
   t.scores = a->scores;
   t.ctx = a->dctx;
   LAUNCH(c, K_ATTENTION, launch_attention_core(t, c->stream));

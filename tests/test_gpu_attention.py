@@ -158,11 +158,12 @@ def test_attention_long_context(ctx, nh, nkv, hd):
     att.close()
 
 
-@pytest.mark.parametrize("nh,nkv,hd,steps", [(2, 1, 80, 2060), (3, 1, 48, 520), (2, 2, 16, 4100)])
+@pytest.mark.parametrize("nh,nkv,hd,steps", [(2, 1, 80, 2060), (3, 1, 272, 600), (2, 2, 16, 4100)])
 def test_attention_softmax_context_edges(ctx, nh, nkv, hd, steps):
     # both sides of the row lengths that pick the values per lane of the
     # ordered sum, of the 128-position tiles and of their 64-position batches,
-    # with head sizes whose last column block is half full
+    # and of the rows that one launch takes (512), with head sizes whose last
+    # column block is half full and whose keys fill several chunks of 64
     ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=hd, qk_norm=True, max_len=steps)
     edges = {n - 1 for c in (1, 32, 64, 128, 192, 256, 384, 512, 1024, 2048, 4096) for n in (c, c + 1, c + 2)}
     for pos in range(steps):
