@@ -117,6 +117,14 @@ struct DownArgs {
   // routes or combine): x (f32, 16-byte aligned) quantized by the kernel,
   // or hact when null
   const float* x;
+  // launch_matvec_many: further matrices of the same row length and x;
+  // work-groups from more[i].first on take matrix i + 1
+  struct {
+    const uint8_t* codes;
+    const uint16_t* scales;
+    float* out;
+    int rows, first;
+  } more[2];
 };
 
 hipError_t launch_down_combine(int dtype, const DownArgs& a, hipStream_t st);
@@ -141,6 +149,11 @@ struct MatvecArgs {
   const uint16_t* scales2;
 };
 hipError_t launch_matvec(int dtype, const MatvecArgs& a, hipStream_t st);
+// Two or three matrices of one dtype and row length and the same x (f32,
+// 16-byte aligned) in one launch, each with its own rows and out; whether it
+// takes them (then x is quantized in the kernel, and a.act is not read).
+bool matvec_takes_many(int nb, int n, const size_t* rows);
+hipError_t launch_matvec_many(int dtype, int n, const MatvecArgs* a, hipStream_t st);
 // Whether launch_matvec takes x (f32, 16-byte aligned) for rows of nb
 // blocks, quantizing it in the kernel; otherwise the caller quantizes x
 // into act first.
@@ -222,6 +235,11 @@ hipError_t launch_stream_read(const void* src, size_t n16, unsigned workgroups, 
 // aligned), in the reference's 8-lane dot order.
 hipError_t launch_gemv_float(int dtype, const void* w, const float* x, size_t rows, size_t cols,
                              float* out, hipStream_t st);
+// The same for n matrices (at most MATVEC_MANY) of one dtype and row length
+// and one x, in one launch: out[i][rows[i]] = w[i] x.
+constexpr int MATVEC_MANY = 3;
+hipError_t launch_gemv_float_many(int dtype, int n, const void* const* w, const float* x, const size_t* rows,
+                                  size_t cols, float* const* out, hipStream_t st);
 // out[r] = rms_norm(x[r] (+ delta[r], stored back into x), w) for each of
 // `rows` rows of n values (n <= 8192)
 hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t rows, size_t n,

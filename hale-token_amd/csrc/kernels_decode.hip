@@ -1659,9 +1659,23 @@ __global__ __launch_bounds__(64 * NW) void k_down_tile(DownArgs a) {
   // get ids of one residue class when the grid allows (they share the
   // tile's scale lines).
   constexpr int PER_TILE = 32 / RW;
-  const int g = blockIdx.x;
+  int g = blockIdx.x, groups = gridDim.x;
+  if constexpr (PLAIN) {  // of several matrices, this work-group's
+    if (a.more[0].codes) {  // uniform
+      const int second = a.more[0].first, third = a.more[1].codes ? a.more[1].first : groups;
+      const int m = g < second ? 0 : (g < third ? 1 : 2);
+      groups = m == 0 ? second : (m == 1 ? third - second : groups - third);
+      if (m) {
+        g -= m == 1 ? second : third;
+        a.codes = m == 1 ? a.more[0].codes : a.more[1].codes;
+        a.scales = m == 1 ? a.more[0].scales : a.more[1].scales;
+        a.out = m == 1 ? a.more[0].out : a.more[1].out;
+        a.rows = m == 1 ? a.more[0].rows : a.more[1].rows;
+      }
+    }
+  }
   size_t row0 = (size_t)g * RW;
-  if (PER_TILE > 1 && gridDim.x % (8 * PER_TILE) == 0) {
+  if (PER_TILE > 1 && groups % (8 * PER_TILE) == 0) {
     const int gx = g & 7, gj = g >> 3;
     row0 = (size_t)(gx + 8 * (gj / PER_TILE)) * TILE + (size_t)(gj % PER_TILE) * RW;
   }
@@ -2691,6 +2705,58 @@ static bool matvec_spread(int nb, size_t rows) {
 
 bool matvec_takes_x(int nb, size_t rows) { return nb <= MATVEC_XQ_MAX_NB || matvec_spread(nb, rows); }
 
+// k_down_tile's plain form over n matrices of one row length and x; rows per
+// work-group as for one matrix of all their rows.
+static hipError_t launch_spread(int dtype, int n, const MatvecArgs* a, hipStream_t st) {
+  DownArgs d{};
+  d.codes = a[0].codes;
+  d.scales = a[0].scales;
+  d.nb = a[0].nb;
+  d.rows = a[0].rows;
+  d.hact = a[0].act;
+  d.slots = 1;
+  d.out = a[0].out;
+  d.tokens = 1;
+  d.x = a[0].x;
+  size_t prow = 0;
+  for (int i = 0; i < n; i++) prow += padded_rows((size_t)a[i].rows);
+  auto busiest = [&](size_t rw) { return (prow / rw + 255) / 256 * rw; };
+  const bool half = busiest(16) < busiest(32);
+  size_t first = 0;
+  for (int i = 1; i < n; i++) {
+    first += padded_rows((size_t)a[i - 1].rows) / (half ? 16 : 32);
+    d.more[i - 1] = {a[i].codes, a[i].scales, a[i].out, a[i].rows, (int)first};
+  }
+  const dim3 grid((unsigned)(prow / (half ? 16 : 32)));
+  const uint32_t lds = (uint32_t)down_tile_lds(1, d.nb);
+  if (half && dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 16, 1, true>, grid, 1024, lds, st, d);
+  if (half) return launch(k_down_tile<Q4_0, 1, 16, 16, 2, true>, grid, 1024, lds, st, d);
+  if (dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 32, 1, true>, grid, 1024, lds, st, d);
+  return launch(k_down_tile<Q4_0, 1, 16, 32, 2, true>, grid, 1024, lds, st, d);
+}
+
+// The spread form's shapes, for each matrix alone and for their rows together
+// (as many as one matrix may have).
+bool matvec_takes_many(int nb, int n, const size_t* rows) {
+  size_t all = 0;
+  for (int i = 0; i < n; i++) {
+    if (!matvec_spread(nb, rows[i])) return false;
+    all += rows[i];
+  }
+  return n >= 2 && n <= MATVEC_MANY && matvec_spread(nb, all);
+}
+
+hipError_t launch_matvec_many(int dtype, int n, const MatvecArgs* a, hipStream_t st) {
+  size_t rows[MATVEC_MANY] = {};
+  if ((dtype != Q8_0 && dtype != Q4_0) || n < 2 || n > MATVEC_MANY) return hipErrorInvalidValue;
+  for (int i = 0; i < n; i++) {
+    if (a[i].nb != a[0].nb || a[i].x != a[0].x || a[i].rows < 1) return hipErrorInvalidValue;
+    rows[i] = (size_t)a[i].rows;
+  }
+  if (!a[0].x || ((uintptr_t)a[0].x & 15) || !matvec_takes_many(a[0].nb, n, rows)) return hipErrorNotSupported;
+  return launch_spread(dtype, n, a, st);
+}
+
 hipError_t launch_matvec(int dtype, const MatvecArgs& a, hipStream_t st) {
   if (a.nb < 1 || a.rows < 1) return hipErrorInvalidValue;
   if (dtype != Q8_0 && dtype != Q4_0) return hipErrorInvalidValue;
@@ -2703,27 +2769,8 @@ hipError_t launch_matvec(int dtype, const MatvecArgs& a, hipStream_t st) {
   // kernel (rows of up to 512 blocks), no quantization launch before it;
   // 768 x 2048 q8_0 3.8 -> 3.4).  Rows of 24 blocks (2048 x 768: 3.06 against 3.23-3.48 us) and
   // 151,936 rows (51.9 against 52.5-53.8 us) stay on the chain kernel.
-  if (matvec_spread(a.nb, (size_t)a.rows) && (xq ? ((uintptr_t)a.x & 15) == 0 : a.act != nullptr)) {
-    DownArgs d{};
-    d.codes = a.codes;
-    d.scales = a.scales;
-    d.nb = a.nb;
-    d.rows = a.rows;
-    d.hact = a.act;
-    d.slots = 1;
-    d.out = a.out;
-    d.tokens = 1;
-    d.x = a.x;
-    const size_t prow = padded_rows((size_t)a.rows);
-    auto busiest = [&](size_t rw) { return (prow / rw + 255) / 256 * rw; };
-    const bool half = busiest(16) < busiest(32);
-    const dim3 grid((unsigned)(prow / (half ? 16 : 32)));
-    const uint32_t lds = (uint32_t)down_tile_lds(1, a.nb);
-    if (half && dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 16, 1, true>, grid, 1024, lds, st, d);
-    if (half) return launch(k_down_tile<Q4_0, 1, 16, 16, 2, true>, grid, 1024, lds, st, d);
-    if (dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 32, 1, true>, grid, 1024, lds, st, d);
-    return launch(k_down_tile<Q4_0, 1, 16, 32, 2, true>, grid, 1024, lds, st, d);
-  }
+  if (matvec_spread(a.nb, (size_t)a.rows) && (xq ? ((uintptr_t)a.x & 15) == 0 : a.act != nullptr))
+    return launch_spread(dtype, 1, &a, st);
   if (xq && (((uintptr_t)a.x & 15) || a.nb > MATVEC_XQ_MAX_NB)) return hipErrorNotSupported;
   if (!xq && (!a.act || a.nb > MATVEC_MAX_NB)) return hipErrorNotSupported;
   const size_t prow = padded_rows((size_t)a.rows);

@@ -56,12 +56,26 @@ __device__ __forceinline__ void unpack16(const u32x4& v, float* o) {
   }
 }
 
+// The matrices of one launch (all cols long): work-groups first[i] ..
+// first[i + 1] - 1 take matrix i.
+struct FloatMats {
+  const uint8_t* w[MATVEC_MANY];
+  float* out[MATVEC_MANY];
+  int rows[MATVEC_MANY], first[MATVEC_MANY];
+  __device__ __forceinline__ int of(int group) const {
+    int i = 0;
+#pragma unroll
+    for (int j = 1; j < MATVEC_MANY; j++) i = group >= first[j] ? j : i;
+    return i;
+  }
+};
+
 // VEC: every row starts 16-byte aligned, so a piece is one 16-byte load;
-// otherwise it is read value by value.
-template <int DT, bool VEC>
-__global__ __launch_bounds__(256) void k_gemv_float(const uint8_t* __restrict__ w,
-                                                    const float* __restrict__ x, int rows,
-                                                    int cols, float* __restrict__ out) {
+// otherwise it is read value by value.  MANY: several matrices; one alone
+// skips the choice (2 % of a 151,936 x 2048 projection's time).
+template <int DT, bool VEC, bool MANY>
+__global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __restrict__ x,
+                                                    int cols) {
   constexpr int PER = FloatFmt<DT>::PER16;
   constexpr int ESZ = DT == F32 ? 4 : 2;
   constexpr int UPR = FK / PER;          // 16-byte pieces per row of a chunk
@@ -72,7 +86,11 @@ __global__ __launch_bounds__(256) void k_gemv_float(const uint8_t* __restrict__ 
   __shared__ __attribute__((aligned(16))) float prod[2][FR][FK + FPAD];
 
   const int tid = threadIdx.x;
-  const int row0 = blockIdx.x * FR;
+  const int mi = MANY ? m.of((int)blockIdx.x) : 0;
+  const uint8_t* __restrict__ w = m.w[mi];
+  float* __restrict__ out = m.out[mi];
+  const int rows = m.rows[mi];
+  const int row0 = ((int)blockIdx.x - m.first[mi]) * FR;
   const int done = cols / 8 * 8;         // columns covered by the lane accumulators
   const int nchunks = (done + FK - 1) / FK;
   const size_t rb = (size_t)cols * ESZ;  // row bytes
@@ -213,17 +231,34 @@ hipError_t launch_encode_half(int dtype, const float* values, size_t n, void* ou
 
 hipError_t launch_gemv_float(int dtype, const void* w, const float* x, size_t rows, size_t cols,
                              float* out, hipStream_t st) {
-  if (rows == 0) return hipSuccess;
-  if (rows > (size_t)INT32_MAX - FR || cols > (size_t)INT32_MAX - FK) return hipErrorInvalidValue;
+  return launch_gemv_float_many(dtype, 1, &w, x, &rows, cols, &out, st);
+}
+
+hipError_t launch_gemv_float_many(int dtype, int n, const void* const* w, const float* x, const size_t* rows,
+                                  size_t cols, float* const* out, hipStream_t st) {
+  if (n < 1 || n > MATVEC_MANY || cols > (size_t)INT32_MAX - FK) return hipErrorInvalidValue;
   if ((uintptr_t)x % 16) return hipErrorInvalidValue;  // x is read in 16-byte pieces
-  const unsigned grid = (unsigned)((rows + FR - 1) / FR);
-  const uint8_t* wb = (const uint8_t*)w;
   const int esz = dtype == F32 ? 4 : 2;
-  const bool vec = (cols * esz) % 16 == 0 && (uintptr_t)w % 16 == 0;
-#define HALE_FLOAT_CASE(D)                                                                          \
-  if (dtype == D)                                                                                 \
-    return vec ? launch(k_gemv_float<D, true>, grid, 256, 0, st, wb, x, (int)rows, (int)cols, out) \
-               : launch(k_gemv_float<D, false>, grid, 256, 0, st, wb, x, (int)rows, (int)cols, out);
+  bool vec = (cols * esz) % 16 == 0;
+  FloatMats m{};
+  size_t groups = 0;
+  for (int i = 0; i < MATVEC_MANY; i++) {
+    m.first[i] = i < n ? (int)groups : INT32_MAX;
+    if (i >= n) continue;
+    if (rows[i] > (size_t)INT32_MAX - FR) return hipErrorInvalidValue;
+    m.w[i] = (const uint8_t*)w[i];
+    m.out[i] = out[i];
+    m.rows[i] = (int)rows[i];
+    vec = vec && (uintptr_t)w[i] % 16 == 0;
+    groups += (rows[i] + FR - 1) / FR;
+    if (groups > (size_t)INT32_MAX) return hipErrorInvalidValue;
+  }
+  if (groups == 0) return hipSuccess;
+  auto run = [&](auto kernel) { return launch(kernel, (unsigned)groups, 256, 0, st, m, x, (int)cols); };
+#define HALE_FLOAT_CASE(D)                                                        \
+  if (dtype == D)                                                                 \
+    return vec ? (n > 1 ? run(k_gemv_float<D, true, true>) : run(k_gemv_float<D, true, false>)) \
+               : (n > 1 ? run(k_gemv_float<D, false, true>) : run(k_gemv_float<D, false, false>));
   HALE_FLOAT_CASE(F32)
   HALE_FLOAT_CASE(F16)
   HALE_FLOAT_CASE(BF16)

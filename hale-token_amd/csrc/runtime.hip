@@ -836,6 +836,30 @@ static int matvec_enqueue(hale_ctx* c, const hale_matrix* m, const float* dx, fl
   return HALE_OK;
 }
 
+// matvec_enqueue of three matrices on the same dx (Attention::forward's q, k
+// and v): one launch when they share a dtype and row length that the kernels
+// take together, else one after the other.
+static int matvec3_enqueue(hale_ctx* c, const hale_matrix* const (&m)[3], const float* dx, float* const (&dout)[3],
+                           ActBlock* act) {
+  const bool alike = m[0]->dtype == m[1]->dtype && m[0]->dtype == m[2]->dtype && m[0]->cols == m[1]->cols &&
+                     m[0]->cols == m[2]->cols && ((uintptr_t)dx & 15) == 0;
+  const size_t rows[3] = {m[0]->rows, m[1]->rows, m[2]->rows}, nb = m[0]->cols / HALE_QK;
+  if (alike && !quantized(m[0]->dtype)) {
+    const void* w[3] = {m[0]->raw, m[1]->raw, m[2]->raw};
+    LAUNCH(c, K_GEMV, launch_gemv_float_many(m[0]->dtype, 3, w, dx, rows, m[0]->cols, dout, c->stream));
+    return HALE_OK;
+  }
+  if (alike && quantized(m[0]->dtype) && matvec_takes_many((int)nb, 3, rows)) {
+    MatvecArgs a[3];
+    for (int i = 0; i < 3; i++) a[i] = MatvecArgs{m[i]->codes, m[i]->scales, (int)nb, (int)rows[i], dx, nullptr, dout[i]};
+    LAUNCH(c, K_GEMV, launch_matvec_many(m[0]->dtype, 3, a, c->stream));
+    return HALE_OK;
+  }
+  for (int i = 0; i < 3; i++)
+    if (int rc = matvec_enqueue(c, m[i], dx, dout[i], act)) return rc;
+  return HALE_OK;
+}
+
 extern "C" int hale_matvec(hale_ctx* c, const hale_matrix* m, const float* x, size_t xlen,
                            float* out, size_t outlen) {
   if (!c || !m || !x || !out) return fail(c, HALE_EINVAL, "matvec: NULL argument");
@@ -2328,9 +2352,7 @@ extern "C" int hale_attention_forward_device(hale_attention* a, const float* d_x
     return fail(c, HALE_EINVAL, "context overflow: %zu positions needed, the cache holds %zu",
                 position + 1, a->max_len);
   HIPCHK(c, hipSetDevice(c->device));
-  int rc = matvec_enqueue(c, a->q, d_x, a->dq, a->act);
-  if (!rc) rc = matvec_enqueue(c, a->k, d_x, a->dk, a->act);
-  if (!rc) rc = matvec_enqueue(c, a->v, d_x, a->dv, a->act);
+  int rc = matvec3_enqueue(c, {a->q, a->k, a->v}, d_x, {a->dq, a->dk, a->dv}, a->act);
   if (rc) return rc;
   AttnArgs t{};
   t.q = a->dq;

@@ -140,6 +140,23 @@ def test_attention_decode_bit_exact(ctx, dtype, Hd, nh, nkv, hd, qk, steps):
     att.close()
 
 
+@pytest.mark.parametrize("dtype,Hd,nh,nkv,hd", [
+    (O.Q8_0, 1024, 6, 2, 80),    # 480 and 160 rows: padded to 512 and 192, three matrices in one launch
+    (O.Q4_0, 1056, 4, 2, 48),    # 33-block rows, 96-row key and value matrices
+    (O.Q8_0, 4096, 32, 8, 128),  # 6144 rows: 32-row work-groups for all three
+    (O.Q4_0, 512, 4, 2, 64),     # 16-block rows: one launch each
+    (O.F16, 260, 3, 1, 80),      # rows that no 16-byte piece divides
+    (O.F32, 64, 5, 5, 16),       # 80 rows each: ten work-groups per matrix
+])
+def test_attention_projections_together(ctx, dtype, Hd, nh, nkv, hd):
+    ref, att = build(ctx, dtype, Hd, nh, nkv, hd, seed=Hd + hd, qk_norm=False, max_len=4)
+    for pos in range(4):
+        x = O.normal(700 + pos, Hd)
+        c, s = O.rope_angles(hd, 1e6, pos)
+        assert same_bits(att.forward(x, pos, c, s), ref.forward(x, c, s)), pos
+    att.close()
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 32), (16, 2, 16), (16, 1, 16), (6, 2, 16), (4, 4, 16)])
 def test_attention_long_context(ctx, nh, nkv, hd):
     # 1100 positions with GQA groups of 4, 8, 16, 3 and 1: 35 score blocks of
