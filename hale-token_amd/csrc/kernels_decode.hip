@@ -96,10 +96,9 @@ __device__ __forceinline__ uint16_t ld_u16(const uint8_t* p) { return (uint16_t)
 
 // decode_row over n values of reference-layout rows laid end to end (a row's
 // blocks follow the previous row's, so value i is block i / 32, position
-// i % 32 of the run).  One thread per value.  A: the base is aligned to the
-// dtype's element or scale size, so values and scales load whole;
-// otherwise by bytes, as the reference's unaligned fallback reads them.
-template <int DT, bool A>
+// i % 32 of the run): any base, one thread per value, elements and scales by
+// bytes as the reference's unaligned fallback reads them.
+template <int DT>
 __global__ __launch_bounds__(256) void k_decode_ref(const uint8_t* __restrict__ src, size_t n,
                                                     float* __restrict__ out) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
@@ -107,18 +106,16 @@ __global__ __launch_bounds__(256) void k_decode_ref(const uint8_t* __restrict__ 
   float v;
   if constexpr (DT == F32) {
     const uint8_t* p = src + 4 * i;
-    const unsigned u = A ? *(const unsigned*)p
-                         : (unsigned)p[0] | (unsigned)p[1] << 8 | (unsigned)p[2] << 16 | (unsigned)p[3] << 24;
-    v = __uint_as_float(u);
+    v = __uint_as_float((unsigned)p[0] | (unsigned)p[1] << 8 | (unsigned)p[2] << 16 | (unsigned)p[3] << 24);
   } else if constexpr (DT == F16) {
-    v = h2f_quiet(A ? ((const uint16_t*)src)[i] : ld_u16(src + 2 * i));
+    v = h2f_quiet(ld_u16(src + 2 * i));
   } else if constexpr (DT == BF16) {
-    v = __uint_as_float((unsigned)(A ? ((const uint16_t*)src)[i] : ld_u16(src + 2 * i)) << 16);
+    v = __uint_as_float((unsigned)ld_u16(src + 2 * i) << 16);
   } else {
     constexpr int BB = DT == Q8_0 ? 34 : 18;
     const uint8_t* blk = src + (i / QK) * BB;
     const int j = (int)(i % QK);
-    const float scale = h2f_quiet(A ? *(const uint16_t*)blk : ld_u16(blk));
+    const float scale = h2f_quiet(ld_u16(blk));
     if constexpr (DT == Q8_0) {
       v = scale * (float)(int8_t)blk[2 + j];
     } else {
@@ -127,6 +124,72 @@ __global__ __launch_bounds__(256) void k_decode_ref(const uint8_t* __restrict__ 
     }
   }
   out[i] = v;
+}
+
+// The same for a source aligned to its element or scale (2 or 4 bytes) and a
+// 16-byte aligned output: 16-byte stores, CONV_U pieces per thread in flight.
+// A piece is 4 values, for q4_0 the 4 + 4 whose codes share four bytes.
+// HBM-bound by the f32 side; 4096 x 14336 q4_0: 105 us with one value per
+// thread, 40 us so.
+constexpr int CONV_U = 4;
+
+template <int DT>
+__global__ __launch_bounds__(256) void k_decode_vec(const uint8_t* __restrict__ src, size_t n,
+                                                    float* __restrict__ out) {
+  constexpr int PER = DT == Q4_0 ? 8 : 4;  // values per piece
+  const size_t pieces = n / PER;
+  const size_t p0 = (size_t)blockIdx.x * (256 * CONV_U) + threadIdx.x;
+  // the piece's codes or elements, loaded whole at their own alignment
+  constexpr int WORDS = DT == F32 ? 4 : (DT == F16 || DT == BF16 ? 2 : 1);
+  struct __attribute__((packed, aligned(DT == F32 ? 4 : 2))) Words {
+    unsigned w[WORDS];
+  } ws[CONV_U];
+  uint16_t sc[CONV_U];
+#pragma unroll
+  for (int u = 0; u < CONV_U; u++) {  // clamped: unconditional loads stay in flight together
+    const size_t p = p0 + 256 * u < pieces ? p0 + 256 * u : pieces - 1;
+    if constexpr (DT == Q8_0 || DT == Q4_0) {
+      constexpr int PPB = QK / PER, BB = DT == Q8_0 ? 34 : 18;
+      const uint8_t* blk = src + p / PPB * BB;
+      sc[u] = *(const uint16_t*)blk;
+      ws[u] = *(const Words*)(blk + 2 + 4 * (p % PPB));
+    } else {
+      ws[u] = ((const Words*)src)[p];
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < CONV_U; u++) {
+    const size_t p = p0 + 256 * u;
+    if (p >= pieces) break;
+    const unsigned w = ws[u].w[0];
+    f32x4 v;
+    if constexpr (DT == Q4_0) {
+      const float scale = h2f_quiet(sc[u]);
+      f32x4 hi;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        v[j] = scale * ((float)(w >> 8 * j & 15u) - 8.0f);
+        hi[j] = scale * ((float)(w >> (8 * j + 4) & 15u) - 8.0f);
+      }
+      float* o = out + p / 4 * QK + 4 * (p % 4);
+      *(f32x4*)o = v;
+      *(f32x4*)(o + 16) = hi;
+    } else {
+      const float scale = DT == Q8_0 ? h2f_quiet(sc[u]) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        if constexpr (DT == Q8_0) {
+          v[j] = scale * (float)(int8_t)(w >> 8 * j);
+        } else if constexpr (DT == F32) {
+          v[j] = __uint_as_float(ws[u].w[j]);
+        } else {
+          const unsigned half = ws[u].w[j / 2] >> 16 * (j & 1);
+          v[j] = DT == F16 ? h2f_quiet((uint16_t)half) : __uint_as_float(half << 16);
+        }
+      }
+      *(f32x4*)(out + 4 * p) = v;
+    }
+  }
 }
 
 // The same values read from the HBM tile planes: rows row0 .. row0 + nrows - 1
@@ -160,59 +223,94 @@ __global__ __launch_bounds__(256) void k_decode_tiles(const uint8_t* __restrict_
 // Weight quantization: encode_row (src/tensor/quant.rs:274-321)
 // ===========================================================================
 
-// One thread per block; writes the reference layout.
-template <int DT>
+// One block from an aligned group of 8 lanes, lane j holding elements 4j..4j+3
+// (16-byte loads, a wave's contiguous), ENC_U blocks per group in flight; writes the
+// reference layout.  HBM-bound by the f32 side; 4096 x 14336 to q4_0: 81 us
+// with one thread per block and byte stores, 64 us so.  OUT: the
+// element the output is aligned to (uint16_t, or bytes at an odd base).
+constexpr int ENC_U = 4;
+
+template <typename OUT>
+__device__ __forceinline__ void store_code_bytes(uint8_t* dst, unsigned v, int n) {
+  OUT* d = (OUT*)dst;
+#pragma unroll
+  for (int i = 0; i < n / (int)sizeof(OUT); i++) d[i] = (OUT)(v >> (8 * sizeof(OUT) * i));
+}
+
+template <int DT, typename OUT>
 __global__ __launch_bounds__(256) void k_encode(const float* __restrict__ values, size_t nblocks,
                                                 uint8_t* __restrict__ out) {
-  size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= nblocks) return;
-  const f32x4* src = (const f32x4*)(values + id * QK);
-  float v[QK];
+  const size_t id0 = (size_t)blockIdx.x * (32 * ENC_U) + threadIdx.x / 8;
+  const int j = threadIdx.x & 7;
+  f32x4 vs[ENC_U];
 #pragma unroll
-  for (int i = 0; i < QK / 4; i++) {
-    f32x4 f = src[i];
-    v[4 * i] = f.x;
-    v[4 * i + 1] = f.y;
-    v[4 * i + 2] = f.z;
-    v[4 * i + 3] = f.w;
+  for (int u = 0; u < ENC_U; u++) {  // clamped: unconditional loads stay in flight together
+    const size_t id = id0 + 32 * u < nblocks ? id0 + 32 * u : nblocks - 1;
+    vs[u] = *(const f32x4*)(values + id * QK + 4 * j);
   }
-  if constexpr (DT == Q8_0) {
-    // encode_block_q8_0, quant.rs:295-305
-    uint8_t* dst = out + id * 34;
-    float amax = 0.0f;
 #pragma unroll
-    for (int j = 0; j < QK; j++) amax = fmaxf(amax, fabsf(v[j]));
-    float scale = amax / 127.0f;
-    float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
-    uint16_t h = f2h(scale);
-    dst[0] = (uint8_t)(h & 0xff);
-    dst[1] = (uint8_t)(h >> 8);
+  for (int u = 0; u < ENC_U; u++) {  // every lane takes part in the exchanges
+    const size_t id = id0 + 32 * u;
+    const f32x4 v = vs[u];
+    unsigned codes = 0;
+    if constexpr (DT == Q8_0) {
+      // encode_block_q8_0, quant.rs:295-305
+      // magnitudes as integers: ordered as the floats are, NaN above all
+      unsigned top = 0;
 #pragma unroll
-    for (int j = 0; j < QK; j++) {
-      float r = roundf(v[j] * inv);
-      r = r < -127.0f ? -127.0f : r;  // f32::clamp keeps NaN, `as i8` maps it to 0
-      r = r > 127.0f ? 127.0f : r;
-      dst[2 + j] = (uint8_t)(int8_t)sat_i8(r);
-    }
-  } else {
-    // encode_block_q4_0, quant.rs:309-321
-    uint8_t* dst = out + id * 18;
-    float extreme = 0.0f;
+      for (int i = 0; i < 4; i++) top = max(top, __float_as_uint(v[i]) & 0x7fffffffu);
+      top = max(top, (unsigned)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xF, 0xF, false));   // lane ^ 1
+      top = max(top, (unsigned)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xF, 0xF, false));   // lane ^ 2
+      top = max(top, (unsigned)__builtin_amdgcn_update_dpp(0, (int)top, 0x141, 0xF, 0xF, false));  // mirror of 8
+      float amax = __uint_as_float(top);
+      if (__any(top > 0x7f800000u)) {
+        // a NaN: the maximum as it folds in order (a quiet one is skipped, a
+        // signalling one becomes the maximum and gives way to the next value)
+        float m = 0.0f;
+        for (int from = 0; from < 8; from++)
 #pragma unroll
-    for (int j = 0; j < QK; j++)
-      if (fabsf(v[j]) > fabsf(extreme)) extreme = v[j];
-    float scale = extreme / -8.0f;
-    float inv = scale != 0.0f ? 1.0f / scale : 0.0f;
-    uint16_t h = f2h(scale);
-    dst[0] = (uint8_t)(h & 0xff);
-    dst[1] = (uint8_t)(h >> 8);
+          for (int i = 0; i < 4; i++) m = fmaxf(m, fabsf(__shfl(v[i], from, 8)));
+        amax = top > 0x7f800000u ? m : amax;
+      }
+      const float scale = amax / 127.0f;
+      const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
 #pragma unroll
-    for (int j = 0; j < QK / 2; j++) {
-      int lo = sat_i32(v[j] * inv + 8.5f);
-      int hi = sat_i32(v[j + QK / 2] * inv + 8.5f);
-      lo = lo < 0 ? 0 : (lo > 15 ? 15 : lo);
-      hi = hi < 0 ? 0 : (hi > 15 ? 15 : hi);
-      dst[2 + j] = (uint8_t)(lo | (hi << 4));
+      for (int i = 0; i < 4; i++) {
+        float r = roundf(v[i] * inv);
+        r = r == r ? fminf(fmaxf(r, -127.0f), 127.0f) : 0.0f;  // f32::clamp keeps NaN, `as i8` maps it to 0
+        codes |= (unsigned)((int)r & 0xff) << 8 * i;
+      }
+      if (id < nblocks) {
+        uint8_t* dst = out + id * 34;
+        if (j == 0) store_code_bytes<OUT>(dst, f2h(scale), 2);
+        store_code_bytes<OUT>(dst + 2 + 4 * j, codes, 4);
+      }
+    } else {
+      // encode_block_q4_0, quant.rs:309-321: the first of the largest
+      float extreme = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (fabsf(v[i]) > fabsf(extreme)) extreme = v[i];
+      auto join = [&](float other, bool earlier) {  // the other lanes' extreme
+        if (earlier ? fabsf(other) >= fabsf(extreme) : fabsf(other) > fabsf(extreme)) extreme = other;
+      };
+      join(HALE_DPP_F32(extreme, 0xB1), j & 1);
+      join(HALE_DPP_F32(extreme, 0x4E), j & 2);
+      join(HALE_DPP_F32(extreme, 0x141), j & 4);
+      const float scale = extreme / -8.0f;
+      const float inv = scale != 0.0f ? 1.0f / scale : 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        // truncated and clamped to 0 .. 15, a NaN to 0 (the maximum skips it)
+        codes |= (unsigned)fminf(fmaxf(v[i] * inv + 8.5f, 0.0f), 15.0f) << 8 * i;
+      }
+      // lanes 0-3 hold the low nibbles, lanes 4-7 the high ones
+      codes |= (unsigned)__builtin_amdgcn_update_dpp(0, (int)codes, 0x104, 0xF, 0xF, false) << 4;
+      if (id < nblocks && j < 4) {
+        uint8_t* dst = out + id * 18;
+        if (j == 0) store_code_bytes<OUT>(dst, f2h(scale), 2);
+        store_code_bytes<OUT>(dst + 2 + 4 * j, codes, 4);
+      }
     }
   }
 }
@@ -2384,13 +2482,27 @@ hipError_t launch_unpack(int dtype, const uint8_t* codes, const uint16_t* scales
 
 hipError_t launch_decode_ref(int dtype, const void* src, size_t n, float* out, hipStream_t st) {
   if (n == 0) return hipSuccess;
-  const unsigned grid = (unsigned)((n + 255) / 256);
   const uint8_t* b = (const uint8_t*)src;
-  const bool a = (uintptr_t)src % (dtype == F32 ? 4 : 2) == 0;
-#define HALE_DECODE_REF(D)                                                            \
-  if (dtype == D)                                                                     \
-    return a ? launch(k_decode_ref<D, true>, grid, 256, 0, st, b, n, out)            \
-             : launch(k_decode_ref<D, false>, grid, 256, 0, st, b, n, out);
+  // whole pieces by 16-byte stores; what is left and other alignments value
+  // by value
+  const size_t per = dtype == Q4_0 ? 8 : 4;
+  if (n >= per && (uintptr_t)src % (dtype == F32 ? 4 : 2) == 0 && (uintptr_t)out % 16 == 0) {
+    const size_t done = n / per * per;
+    const unsigned grid = blocks_for(done / per, 256 * CONV_U);
+    hipError_t e = hipErrorInvalidValue;
+    if (dtype == F32) e = launch(k_decode_vec<F32>, grid, 256, 0, st, b, done, out);
+    if (dtype == F16) e = launch(k_decode_vec<F16>, grid, 256, 0, st, b, done, out);
+    if (dtype == BF16) e = launch(k_decode_vec<BF16>, grid, 256, 0, st, b, done, out);
+    if (dtype == Q8_0) e = launch(k_decode_vec<Q8_0>, grid, 256, 0, st, b, done, out);
+    if (dtype == Q4_0) e = launch(k_decode_vec<Q4_0>, grid, 256, 0, st, b, done, out);
+    if (e != hipSuccess || done == n) return e;
+    b += (dtype == F32 ? 4 : 2) * done;  // only float formats leave a remainder
+    out += done;
+    n -= done;
+  }
+  const unsigned grid = blocks_for(n, 256);
+#define HALE_DECODE_REF(D) \
+  if (dtype == D) return launch(k_decode_ref<D>, grid, 256, 0, st, b, n, out);
   HALE_DECODE_REF(F32)
   HALE_DECODE_REF(F16)
   HALE_DECODE_REF(BF16)
@@ -2415,8 +2527,13 @@ hipError_t launch_decode_tiles(int dtype, const uint8_t* codes, const uint16_t* 
 hipError_t launch_encode(int dtype, const float* values, size_t nblocks, uint8_t* out,
                          hipStream_t st) {
   if (nblocks == 0) return hipSuccess;
-  if (dtype == Q8_0) return launch(k_encode<Q8_0>, blocks_for(nblocks, 256), 256, 0, st, values, nblocks, out);
-  return launch(k_encode<Q4_0>, blocks_for(nblocks, 256), 256, 0, st, values, nblocks, out);
+  const unsigned grid = blocks_for(nblocks, 32 * ENC_U);
+  const bool even = (uintptr_t)out % 2 == 0;
+  if (dtype == Q8_0)
+    return even ? launch(k_encode<Q8_0, uint16_t>, grid, 256, 0, st, values, nblocks, out)
+                : launch(k_encode<Q8_0, uint8_t>, grid, 256, 0, st, values, nblocks, out);
+  return even ? launch(k_encode<Q4_0, uint16_t>, grid, 256, 0, st, values, nblocks, out)
+              : launch(k_encode<Q4_0, uint8_t>, grid, 256, 0, st, values, nblocks, out);
 }
 
 hipError_t launch_act_quant(const float* x, size_t nblocks, ActBlock* act, hipStream_t st) {

@@ -196,37 +196,67 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
 // f16::from_f32 / bf16::from_f32, round to nearest even; a NaN keeps its
 // sign and top payload bits and becomes quiet.
 template <int DT>
+__device__ __forceinline__ uint16_t encode_half(float f) {
+  const unsigned x = __float_as_uint(f);
+  const bool nan = (x & 0x7fffffffu) > 0x7f800000u;
+  if constexpr (DT == F16) {
+    if (nan) return (uint16_t)(((x >> 16) & 0x8000u) | 0x7e00u | ((x & 0x7fffffu) >> 13));
+    return f2h(f);  // v_cvt_f16_f32: round to nearest even, subnormals kept
+  } else {
+    if (nan) return (uint16_t)((x >> 16) | 0x0040u);
+    unsigned q = x >> 16;
+    const unsigned rem = x & 0xffffu;
+    if (rem > 0x8000u || (rem == 0x8000u && (q & 1u))) q++;  // may carry into inf
+    return (uint16_t)q;
+  }
+}
+
+// One value per thread: any alignment, and the last n % 4.
+template <int DT>
 __global__ __launch_bounds__(256) void k_encode_half(const float* __restrict__ v, size_t n,
                                                      uint16_t* __restrict__ out) {
   const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const float f = v[i];
-  const unsigned x = __float_as_uint(f);
-  uint16_t h;
-  if constexpr (DT == F16) {
-    if ((x & 0x7fffffffu) > 0x7f800000u)
-      h = (uint16_t)(((x >> 16) & 0x8000u) | 0x7e00u | ((x & 0x7fffffu) >> 13));
-    else
-      h = f2h(f);  // v_cvt_f16_f32: round to nearest even, subnormals kept
-  } else {
-    if ((x & 0x7fffffffu) > 0x7f800000u) {
-      h = (uint16_t)((x >> 16) | 0x0040u);
-    } else {
-      unsigned q = x >> 16;
-      const unsigned rem = x & 0xffffu;
-      if (rem > 0x8000u || (rem == 0x8000u && (q & 1u))) q++;  // may carry into inf
-      h = (uint16_t)q;
-    }
+  if (i < n) out[i] = encode_half<DT>(v[i]);
+}
+
+// Four values per thread and step (values 16-byte, out 8-byte aligned),
+// HALF_U steps in flight.
+constexpr int HALF_U = 4;
+template <int DT>
+__global__ __launch_bounds__(256) void k_encode_half4(const float* __restrict__ v, size_t pieces,
+                                                      uint16_t* __restrict__ out) {
+  const size_t p0 = (size_t)blockIdx.x * (256 * HALF_U) + threadIdx.x;
+  f32x4 x[HALF_U];
+#pragma unroll
+  for (int u = 0; u < HALF_U; u++) x[u] = ((const f32x4*)v)[p0 + 256 * u < pieces ? p0 + 256 * u : pieces - 1];
+#pragma unroll
+  for (int u = 0; u < HALF_U; u++) {
+    const size_t p = p0 + 256 * u;
+    if (p >= pieces) break;
+    uint64_t w = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) w |= (uint64_t)encode_half<DT>(x[u][j]) << 16 * j;
+    ((uint64_t*)out)[p] = w;
   }
-  out[i] = h;
 }
 
 hipError_t launch_encode_half(int dtype, const float* values, size_t n, void* out, hipStream_t st) {
   if (n == 0) return hipSuccess;
+  if (dtype != F16 && dtype != BF16) return hipErrorInvalidValue;
+  uint16_t* o = (uint16_t*)out;
+  if (n >= 4 && (uintptr_t)values % 16 == 0 && (uintptr_t)out % 8 == 0) {
+    const size_t pieces = n / 4;
+    const unsigned grid = (unsigned)((pieces + 256 * HALF_U - 1) / (256 * HALF_U));
+    const hipError_t e = dtype == F16 ? launch(k_encode_half4<F16>, grid, 256, 0, st, values, pieces, o)
+                                      : launch(k_encode_half4<BF16>, grid, 256, 0, st, values, pieces, o);
+    if (e != hipSuccess || n % 4 == 0) return e;
+    values += 4 * pieces;
+    o += 4 * pieces;
+    n %= 4;
+  }
   const unsigned grid = (unsigned)((n + 255) / 256);
-  if (dtype == F16) return launch(k_encode_half<F16>, grid, 256, 0, st, values, n, (uint16_t*)out);
-  if (dtype == BF16) return launch(k_encode_half<BF16>, grid, 256, 0, st, values, n, (uint16_t*)out);
-  return hipErrorInvalidValue;
+  return dtype == F16 ? launch(k_encode_half<F16>, grid, 256, 0, st, values, n, o)
+                      : launch(k_encode_half<BF16>, grid, 256, 0, st, values, n, o);
 }
 
 hipError_t launch_gemv_float(int dtype, const void* w, const float* x, size_t rows, size_t cols,

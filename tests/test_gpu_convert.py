@@ -110,6 +110,46 @@ def test_decode_every_scale(ctx, dtype):
     assert same_values(got, want, dtype)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 32, 1023, 4096, 4099, 32 * 129, 32 * 4097])
+@pytest.mark.parametrize("in_off,out_off", [(0, 0), (4, 4), (0, 1)])
+def test_device_conversions_at_any_size_and_offset(ctx, dtype, n, in_off, out_off):
+    """Encoding then decoding on the device, values and bytes off their
+    buffers' starts: sizes around the pieces and work-groups of the vector
+    forms, remainders of 1-3 values, bases that only the byte forms take; and
+    nothing is written past either end."""
+    if dtype in QUANT:
+        n = (n + 31) // 32 * 32
+        in_off = 0  # the block encoder takes 16-byte aligned values only
+    elif out_off % 2:
+        out_off *= 4  # half elements stay element-aligned
+    g = np.random.default_rng(n + dtype)
+    v = (g.standard_normal(n) * np.exp(g.uniform(-12, 12, n))).astype(np.float32)
+    v[::7] = np.float32(-0.0)
+    if n >= 64:
+        v[32:64] = g.choice(np.float32([-2.5, 2.5, 1.0]), 32)  # tied extremes: the first wins
+    nb = O.row_bytes(dtype, n) if dtype in QUANT else n * {H.F32: 4, H.F16: 2, H.BF16: 2}[dtype]
+    bv, bb, bo = ctx.malloc(4 * n + 64), ctx.malloc(nb + 64), ctx.malloc(4 * n + 64)
+    bv.upload(np.concatenate([np.zeros(in_off, np.uint8), v.view(np.uint8)]))
+    bb.upload(np.full(nb + 64, 0xA5, np.uint8))
+    bo.upload(np.full(4 * n + 64, 0xA5, np.uint8))
+    L = H.lib()
+    ctx.check(L.hale_encode_rows_device(ctx.handle, dtype, 1, n, H._vp(bv.address + in_off),
+                                        H._vp(bb.address + out_off)), "encode")
+    ctx.check(L.hale_decode_rows_device(ctx.handle, dtype, 1, n, H._vp(bb.address + out_off),
+                                        H._vp(bo.address + 4 * out_off)), "decode")
+    got = bb.download(np.uint8, nb + 64)
+    want = O.encode_matrix(dtype, v.reshape(1, n)).view(np.uint8).reshape(-1)
+    assert (got[out_off:out_off + nb] == want).all()
+    assert (got[:out_off] == 0xA5).all() and (got[out_off + nb:] == 0xA5).all()
+    back = bo.download(np.uint8, 4 * n + 64)
+    vals = back[4 * out_off:4 * out_off + 4 * n].copy().view(np.float32)
+    assert same_values(vals, O.decode_row(dtype, want, n), dtype)
+    assert (back[:4 * out_off] == 0xA5).all() and (back[4 * out_off + 4 * n:] == 0xA5).all()
+    for b in (bv, bb, bo):
+        b.free()
+
+
 def test_decode_rejects_ragged_quantized_rows(ctx):
     """Q8_0 / Q4_0 rows must hold whole blocks (DType::row_bytes)."""
     src, out = np.zeros(64, np.uint8), np.zeros(48, np.float32)
