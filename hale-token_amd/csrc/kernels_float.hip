@@ -14,8 +14,10 @@
 // loads 16-byte pieces of the rows (coalesced along each row) and its x,
 // converts f16/bf16 to f32, and parks the products in LDS; wave 0 then folds
 // them, lane (row r, chain l) reading products 8i + l of row r in order.
-// Two LDS buffers: the next chunk's loads are in flight during a fold.
-// HBM-bound: every weight byte is read once.
+// Two LDS buffers; the loads of up to NS chunks are in flight during a fold.
+// HBM-bound for many rows (151,936 x 2048 bf16: 102-103 us with one chunk in
+// flight, 97.6 us with four: 6.4 TB/s); few rows wait for the round trip and
+// wave 0's fold (5120 x 2048 bf16 8.1 -> 7.4 us).
 #pragma clang fp contract(off)
 
 #include "hale_device.h"
@@ -25,6 +27,7 @@ namespace hale {
 
 constexpr int FR = 8;        // rows per work-group (FR * 8 fold threads, whole waves)
 constexpr int FK = 512;      // columns per chunk
+constexpr int NS = 4;        // chunks in flight
 constexpr int FPAD = 8;      // row pitch FK + FPAD = 8 (mod 64) floats: the fold
                              // threads (row r, chain l) of a wave read banks 8r + l
 
@@ -102,37 +105,33 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
     float x[PER];
   };
   auto load = [&](Regs& R, int ch) {
-    // c is a multiple of PER (4 or 8) and `done` one of 8, so a piece below
-    // `done` ends at or before it; rows past the end are clamped (loaded,
-    // never written)
-    const int c = ch * FK + cpiece;
-    const bool in = c < done;
+    // `done` is a multiple of 8 and PER 4 or 8: pieces past the row's end
+    // repeat the last one, rows past the matrix's the last (loaded, never
+    // written; every load unconditional, so that several chunks stay in
+    // flight)
+    const int c = min(ch * FK + cpiece, done - PER);
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
       const int r = min(row0 + j * RPP + tid / UPR, rows - 1);
       const uint8_t* src = w + (size_t)r * rb + (size_t)c * ESZ;
-      if (in) {
-        if constexpr (VEC) {
-          R.w[j] = __builtin_nontemporal_load((const u32x4*)src);
-        } else if constexpr (DT == F32) {
-          const unsigned* s4 = (const unsigned*)src;
-          R.w[j] = u32x4{s4[0], s4[1], s4[2], s4[3]};
-        } else {
-          const uint16_t* s2 = (const uint16_t*)src;
-          R.w[j] = u32x4{s2[0] | ((unsigned)s2[1] << 16), s2[2] | ((unsigned)s2[3] << 16),
-                         s2[4] | ((unsigned)s2[5] << 16), s2[6] | ((unsigned)s2[7] << 16)};
-        }
+      if constexpr (VEC) {
+        R.w[j] = __builtin_nontemporal_load((const u32x4*)src);
+      } else if constexpr (DT == F32) {
+        const unsigned* s4 = (const unsigned*)src;
+        R.w[j] = u32x4{s4[0], s4[1], s4[2], s4[3]};
+      } else {
+        const uint16_t* s2 = (const uint16_t*)src;
+        R.w[j] = u32x4{s2[0] | ((unsigned)s2[1] << 16), s2[2] | ((unsigned)s2[3] << 16),
+                       s2[4] | ((unsigned)s2[5] << 16), s2[6] | ((unsigned)s2[7] << 16)};
       }
     }
-    if (in) {
 #pragma unroll
-      for (int q = 0; q < PER / 4; q++) {
-        const f32x4 v = *(const f32x4*)(x + c + 4 * q);
-        R.x[4 * q] = v.x;
-        R.x[4 * q + 1] = v.y;
-        R.x[4 * q + 2] = v.z;
-        R.x[4 * q + 3] = v.w;
-      }
+    for (int q = 0; q < PER / 4; q++) {
+      const f32x4 v = *(const f32x4*)(x + c + 4 * q);
+      R.x[4 * q] = v.x;
+      R.x[4 * q + 1] = v.y;
+      R.x[4 * q + 2] = v.z;
+      R.x[4 * q + 3] = v.w;
     }
   };
 
@@ -140,7 +139,8 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
   constexpr int NF = FR * 8;
   const int fr = tid >> 3, fl = tid & 7;
   float acc = 0.0f;
-  auto step = [&](Regs& R, int ch) {
+  // chunk ch from R, which then takes chunk `next` (none: negative)
+  auto step = [&](Regs& R, int ch, int next) {
     const int c0 = ch * FK;
     const int ncols = min(FK, done - c0);
     float(*P)[FK + FPAD] = prod[ch & 1];
@@ -155,12 +155,32 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
       }
     }
     __syncthreads();
-    if (ch + 1 < nchunks) load(R, ch + 1);
+    if (next >= 0) load(R, next);
     if (tid < NF) acc = lds_sum_strided<8>(&P[fr][fl], ncols / 8, acc);
   };
-  Regs R;
-  if (nchunks > 0) load(R, 0);
-  for (int ch = 0; ch < nchunks; ch++) step(R, ch);
+  // NS chunks in flight where a row has as many: one round trip for a row of
+  // 2048 instead of four
+  Regs R[NS];
+  int ch = 0;
+  if (nchunks >= NS) {
+#pragma unroll
+    for (int j = 0; j < NS; j++) {
+      load(R[j], j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (; ch + 2 * NS <= nchunks; ch += NS)
+#pragma unroll
+      for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j);
+#pragma unroll
+    for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j < nchunks ? ch + NS + j : -1);
+    ch += NS;
+#pragma unroll
+    for (int j = 0; j < NS; j++)
+      if (ch + j < nchunks) step(R[j], ch + j, -1);
+  } else if (nchunks > 0) {
+    load(R[0], 0);
+    for (; ch < nchunks; ch++) step(R[0], ch, ch + 1 < nchunks ? ch + 1 : -1);
+  }
 
   if (tid < NF) {
     // reduce (src/tensor/quant.rs:36-40) across the row's 8 chain lanes
