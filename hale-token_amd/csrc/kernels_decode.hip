@@ -479,20 +479,22 @@ __global__ __launch_bounds__(ROUTE_THREADS) void k_route_logits(const float* __r
 }
 
 // The router logits of many tokens (T >= ROUTE_TILED_MIN_T): work-group
-// (eg, tg) computes experts RT_E eg .. RT_E eg + RT_E - 1 (RT_E = 16 or 8)
-// for tokens 8 tg .. 8 tg + 7, one wave per expert.  Lane 8t + l of wave e
-// carries chain l of logit (e, t):
+// (eg, tg) computes RT_E experts from RT_E eg on for 8 TM tokens from 8 TM tg
+// on, EM experts per wave.  Lane 8t + l of a wave carries chain l of its EM
+// experts' logits for tokens t, t + 8, ...:
 // acc = acc + w_e[8s + l] * x_t[8s + l] in order of s, each product rounded
 // before it is added (dot_f32's 8-lane order, quant.rs:152-194).  The
-// RT_E + 8 rows (router rows, then tokens) stream through LDS chain-major in chunks
-// of RT_K steps, two buffers, so chunk c + 1 loads while chunk c is added,
-// and every staged row serves 8 or RT_E logits.  The eight chains of a logit
+// RT_E + 8 TM rows (router rows, then tokens) stream through LDS chain-major in
+// chunks of RT_K steps, two buffers, so chunk c + 1 loads while chunk c is added,
+// and every staged row serves 8 TM or RT_E logits.  The two rounded operations
+// per product bound it; with one logit per lane (EM = TM = 1) every four of
+// them wait for two 16-byte LDS reads, and the reads bound it instead.  Four
+// experts and two tokens per lane read six times per 32 products: 2048 tokens
+// x 128 experts at H 4096 131 -> 94 us.  The eight chains of a logit
 // are reduced in the one-token kernel's fixed order, so each logit has its
 // bits.  Then the work-groups quantize the token tile's activation blocks
 // (as k_act_quant does), each taking its share: block q of the tile goes to
 // the work-group of expert column q % gridDim.x.
-constexpr int RT_T = 8, RT_K = 64;
-constexpr int RT_STRIDE = RT_K + 4;                 // floats per chain row (16-byte aligned)
 // From 48 tokens.  Against one work-group per (expert, token) sized for
 // the row length (eight per CU), per layer, graph replay, row-chain
 // grouped path: Qwen3-30B-A3B q4_0 at 32 / 40 / 48 / 64 / 76 tokens 89.1 /
@@ -501,13 +503,16 @@ constexpr int RT_STRIDE = RT_K + 4;                 // floats per chain row (16-
 // against 289 / 316 / 356.
 constexpr int ROUTE_TILED_MIN_T = 48;
 
-template <int RT_E>  // experts per work-group: one wave each
-__global__ __launch_bounds__(64 * RT_E) void k_route_logits_tiled(const float* __restrict__ router,
-                                                                  const float* __restrict__ x, int H,
-                                                                  int E, int T,
-                                                                  float* __restrict__ logits,
-                                                                  ActBlock* __restrict__ act) {
-  constexpr int NT = 64 * RT_E;                          // threads
+template <int RT_E, int EM, int TM, int RT_K>
+__global__ __launch_bounds__(64 * RT_E / EM) void k_route_logits_tiled(const float* __restrict__ router,
+                                                                       const float* __restrict__ x, int H,
+                                                                       int E, int T,
+                                                                       float* __restrict__ logits,
+                                                                       ActBlock* __restrict__ act) {
+  constexpr int RT_T = 8 * TM;                           // tokens
+  constexpr int UNROLL = EM > 1 ? 4 : 1;                 // LDS reads ahead of the chains
+  constexpr int RT_STRIDE = RT_K + 4;                    // floats per chain row (16-byte aligned)
+  constexpr int NT = 64 * RT_E / EM;                     // threads
   constexpr int RT_BUF = (RT_E + RT_T) * 8 * RT_STRIDE;  // floats per buffer
   __shared__ __attribute__((aligned(16))) float buf[2][RT_BUF];
   const int tid = threadIdx.x;
@@ -544,39 +549,49 @@ __global__ __launch_bounds__(64 * RT_E) void k_route_logits_tiled(const float* _
     }
   };
   const int t = lane >> 3, l = lane & 7;
-  const int wrow = (wave * 8 + l) * RT_STRIDE, xrow = ((RT_E + t) * 8 + l) * RT_STRIDE;
+  const int wrow = (wave * EM * 8 + l) * RT_STRIDE, xrow = ((RT_E + t) * 8 + l) * RT_STRIDE;
   f32x4 v[PPT];
   load_chunk(v, 0);
   store_chunk(v, buf[0]);
   __syncthreads();
-  float acc = 0.0f;
+  float acc[EM][TM] = {};
   for (int c = 0; c < nchunk; c++) {
     if (c + 1 < nchunk) load_chunk(v, c + 1);  // in flight while chunk c is added
     const float* b = buf[c & 1];
     const int kc = min(RT_K, steps - c * RT_K);  // a multiple of 4 (H % 32 == 0)
+#pragma unroll UNROLL
     for (int s4 = 0; s4 < kc; s4 += 4) {
-      const f32x4 wv = *(const f32x4*)(b + wrow + s4);
-      const f32x4 xv = *(const f32x4*)(b + xrow + s4);
-      acc = acc + wv.x * xv.x;
-      acc = acc + wv.y * xv.y;
-      acc = acc + wv.z * xv.z;
-      acc = acc + wv.w * xv.w;
+      f32x4 wv[EM], xv[TM];
+#pragma unroll
+      for (int i = 0; i < EM; i++) wv[i] = *(const f32x4*)(b + wrow + i * 8 * RT_STRIDE + s4);
+#pragma unroll
+      for (int i = 0; i < TM; i++) xv[i] = *(const f32x4*)(b + xrow + i * 64 * RT_STRIDE + s4);
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+#pragma unroll
+        for (int i = 0; i < EM; i++)
+#pragma unroll
+          for (int j = 0; j < TM; j++) acc[i][j] = acc[i][j] + wv[i][q] * xv[j][q];
     }
     if (c + 1 < nchunk) store_chunk(v, buf[(c + 1) & 1]);
     __syncthreads();  // chunk c + 1 staged; every wave is done with chunk c
   }
   const int base = lane & ~7;
-  const float a0 = __shfl(acc, base + 0), a1 = __shfl(acc, base + 1), a2 = __shfl(acc, base + 2),
-              a3 = __shfl(acc, base + 3);
-  const float a4 = __shfl(acc, base + 4), a5 = __shfl(acc, base + 5), a6 = __shfl(acc, base + 6),
-              a7 = __shfl(acc, base + 7);
-  const int e = e0 + wave, tok = t0 + t;
-  if (l == 0 && e < E && tok < T) {
-    const float tail = -0.0f;  // Iterator::sum over the H % 8 leftover products: none (H % 32 == 0)
-    const float s0v = (a0 + a4) + (a1 + a5);
-    const float s1v = (a2 + a6) + (a3 + a7);
-    logits[(size_t)tok * E + e] = (s0v + s1v) + tail;
-  }
+#pragma unroll
+  for (int i = 0; i < EM; i++)
+#pragma unroll
+    for (int j = 0; j < TM; j++) {
+      float a[8];
+#pragma unroll
+      for (int q = 0; q < 8; q++) a[q] = __shfl(acc[i][j], base + q);
+      const int e = e0 + wave * EM + i, tok = t0 + t + 8 * j;
+      if (l == 0 && e < E && tok < T) {
+        const float tail = -0.0f;  // Iterator::sum over the H % 8 leftover products: none (H % 32 == 0)
+        const float s0v = (a[0] + a[4]) + (a[1] + a[5]);
+        const float s1v = (a[2] + a[6]) + (a[3] + a[7]);
+        logits[(size_t)tok * E + e] = (s0v + s1v) + tail;
+      }
+    }
   // this work-group's share of the tile's activation blocks, 8 lanes per
   // block, 128 blocks per pass (the bound is uniform per 8-lane group)
   const int nb = H / QK;
@@ -2425,6 +2440,7 @@ __global__ __launch_bounds__(256) void k_copy(u32x4* __restrict__ dst, const u32
     __builtin_nontemporal_store(__builtin_nontemporal_load(src + i), dst + i);
 }
 
+
 // Plain streaming read, the calibration for what one launch can stream from
 // HBM: work-group g reads a contiguous chunk of src with sixteen 16-byte
 // loads in flight per thread and writes the XOR of every 32-bit word it
@@ -2568,13 +2584,17 @@ hipError_t launch_route_logits(const float* router, const float* x, int H, int E
     // (Qwen3-30B-A3B layer on the row chains at 48 / 64 / 76 tokens: 103.2-
     // 103.6 / 112.7-113.2 / 120.3-120.6 -> 101.8-101.9 / 112.3-112.7 /
     // 118.9-119.3 us per step; Qwen3-235B-A22B at 48: 315-317 -> 310-313)
-    const int tt = (T + RT_T - 1) / RT_T;
-    if ((E + 15) / 16 * tt < 256) {
-      const dim3 grid8((E + 7) / 8, tt);
-      return launch(k_route_logits_tiled<8>, grid8, 512, 0, st, router, x, H, E, T, logits, act);
-    }
-    const dim3 grid((E + 15) / 16, tt);
-    return launch(k_route_logits_tiled<16>, grid, 1024, 0, st, router, x, H, E, T, logits, act);
+    // Register tiles (16 x 16 per work-group of four waves) from 384 of them
+    // on: with one work-group per CU their one wave per SIMD is no faster (500
+    // tokens x 128 experts at H 2048: 24.1 against 21.7 us); 1000 tokens at H
+    // 4096: 73 -> 52 us, 2048 tokens: 131 -> 94 us.
+    const int tt = (T + 7) / 8, et = (E + 15) / 16, tt16 = (T + 15) / 16;
+    if (et * tt16 >= 384)
+      return launch(k_route_logits_tiled<16, 4, 2, 32>, dim3(et, tt16), 256, 0, st, router, x, H, E, T, logits, act);
+    if (et * tt < 256)
+      return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3((E + 7) / 8, tt), 512, 0, st, router, x, H, E, T, logits,
+                    act);
+    return launch(k_route_logits_tiled<16, 1, 1, 64>, dim3(et, tt), 1024, 0, st, router, x, H, E, T, logits, act);
   }
   dim3 grid(E, T);
   if (H <= 8 * ROUTE_THREADS)
@@ -3009,6 +3029,7 @@ hipError_t launch_stream_read(const void* src, size_t n16, unsigned workgroups, 
   if (workgroups < 1 || workgroups > 65535) return hipErrorInvalidValue;
   return launch(k_stream_read, workgroups, 256, 0, st, (const u32x4*)src, n16, out);
 }
+
 
 hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t st) {
   if (!n16) return hipSuccess;

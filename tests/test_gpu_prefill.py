@@ -89,6 +89,18 @@ def test_grouped_router_many_tokens(ctx, dtype, Hd, I, E, k, T):
     moe.close()
 
 
+@pytest.mark.parametrize("dtype,Hd,I,E,k,T", [
+    (H.Q4_0, 288, 32, 1000, 2, 101),  # partial expert and token tiles, a partial chunk (36 steps)
+    (H.Q8_0, 512, 32, 128, 4, 770),   # 8 x 49 tiles, the last token tile of two
+])
+def test_grouped_router_register_tiles(ctx, dtype, Hd, I, E, k, T):
+    """The router's 16 x 16 register tiles (384 of them and more)."""
+    L = O.OracleMoe.synthetic(dtype, Hd, I, E, k, normalize_topk=True, seed=Hd + E + T, with_router=True)
+    moe = make_layer(ctx, L)
+    check(moe, L, O.normal(T + Hd, T * Hd).reshape(T, Hd))
+    moe.close()
+
+
 @pytest.mark.parametrize("dtype,Hd,I,E,k,T,with_router", [
     (H.Q4_0, 256, 96, 32, 4, 40, True),     # 8-block gate/up rows; down rows of 3 blocks (a partial ring cycle)
     (H.Q8_0, 256, 96, 32, 4, 40, False),
