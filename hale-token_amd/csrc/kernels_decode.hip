@@ -226,7 +226,8 @@ __global__ __launch_bounds__(256) void k_decode_tiles(const uint8_t* __restrict_
 // One block from an aligned group of 8 lanes, lane j holding elements 4j..4j+3
 // (16-byte loads, a wave's contiguous), ENC_U blocks per group in flight; writes the
 // reference layout.  HBM-bound by the f32 side; 4096 x 14336 to q4_0: 81 us
-// with one thread per block and byte stores, 64 us so.  OUT: the
+// with one thread per block and byte stores, 64 us so and 43 us with
+// non-temporal loads.  OUT: the
 // element the output is aligned to (uint16_t, or bytes at an odd base).
 constexpr int ENC_U = 4;
 
@@ -246,7 +247,7 @@ __global__ __launch_bounds__(256) void k_encode(const float* __restrict__ values
 #pragma unroll
   for (int u = 0; u < ENC_U; u++) {  // clamped: unconditional loads stay in flight together
     const size_t id = id0 + 32 * u < nblocks ? id0 + 32 * u : nblocks - 1;
-    vs[u] = *(const f32x4*)(values + id * QK + 4 * j);
+    vs[u] = __builtin_nontemporal_load((const f32x4*)(values + id * QK + 4 * j));
   }
 #pragma unroll
   for (int u = 0; u < ENC_U; u++) {  // every lane takes part in the exchanges
