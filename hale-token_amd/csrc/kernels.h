@@ -227,6 +227,8 @@ hipError_t launch_block_sums(int dtype, const uint8_t* codes, const ActBlock* ac
                              size_t cols, int32_t* isums, hipStream_t st);
 hipError_t launch_fill(float* p, size_t n, float v, hipStream_t st);
 hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t st);
+// n 32-bit words between 16-byte aligned buffers
+hipError_t launch_copy_words(void* dst, const void* src, size_t n, hipStream_t st);
 // out[g] = XOR of the 32-bit words of work-group g's contiguous chunk of
 // src[n16] (workgroups in 1..65535)
 hipError_t launch_stream_read(const void* src, size_t n16, unsigned workgroups, unsigned* out,

@@ -2441,6 +2441,15 @@ __global__ __launch_bounds__(256) void k_copy(u32x4* __restrict__ dst, const u32
     __builtin_nontemporal_store(__builtin_nontemporal_load(src + i), dst + i);
 }
 
+__global__ __launch_bounds__(256) void k_copy_words(unsigned* __restrict__ dst, const unsigned* __restrict__ src,
+                                                    size_t n) {
+  const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+  if (i + 4 <= n) {
+    *(u32x4*)(dst + i) = *(const u32x4*)(src + i);
+  } else {
+    for (size_t j = i; j < n; j++) dst[j] = src[j];
+  }
+}
 
 // Plain streaming read, the calibration for what one launch can stream from
 // HBM: work-group g reads a contiguous chunk of src with sixteen 16-byte
@@ -3031,6 +3040,10 @@ hipError_t launch_stream_read(const void* src, size_t n16, unsigned workgroups, 
   return launch(k_stream_read, workgroups, 256, 0, st, (const u32x4*)src, n16, out);
 }
 
+hipError_t launch_copy_words(void* dst, const void* src, size_t n, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  return launch(k_copy_words, blocks_for(n, 1024), 256, 0, st, (unsigned*)dst, (const unsigned*)src, n);
+}
 
 hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t st) {
   if (!n16) return hipSuccess;

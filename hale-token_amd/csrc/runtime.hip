@@ -338,16 +338,35 @@ struct HostStage {
   int reserve(size_t bytes) { return ctx_pinned(c, bytes, &base); }
   int in(void* dev, const void* host, size_t n) {
     std::memcpy(base + used, host, n);
-    const hipError_t e = hipMemcpyAsync(dev, base + used, n, hipMemcpyHostToDevice, c->stream);
+    const hipError_t e = copy(dev, base + used, n, hipMemcpyHostToDevice);
     used += align_up(n, 256);
     return e == hipSuccess ? HALE_OK : fail(c, HALE_EHIP, "copy to device: %s", hipGetErrorString(e));
   }
   int out(void* host, const void* dev, size_t n) {
-    const hipError_t e = hipMemcpyAsync(base + used, dev, n, hipMemcpyDeviceToHost, c->stream);
+    const hipError_t e = copy(base + used, dev, n, hipMemcpyDeviceToHost);
     if (e != hipSuccess) return fail(c, HALE_EHIP, "copy to host: %s", hipGetErrorString(e));
     outs[nouts++] = {host, used, n};
     used += align_up(n, 256);
     return HALE_OK;
+  }
+  // Where a kernel may write a small output itself (the pinned buffer, read
+  // back by finish()); dev, copied by out(), for larger ones.
+  float* direct(void* host, size_t n, float* dev) {
+    if (n > STAGE_SMALL) return dev;
+    outs[nouts++] = {host, used, n};
+    float* p = (float*)(base + used);
+    used += align_up(n, 256);
+    return p;
+  }
+  // Small transfers by a kernel that reads or writes the pinned buffer: the
+  // stream stays on its queue, where a copy command hands over to a copy
+  // engine and back (one q8_0 expert of H 2048, I 768 with its 8 KB in and
+  // out: 27.0 -> 25.3 us).
+  static constexpr size_t STAGE_SMALL = 64 * 1024;
+  hipError_t copy(void* dst, const void* src, size_t n, hipMemcpyKind kind) {
+    if (n <= STAGE_SMALL && n % 4 == 0 && (uintptr_t)dst % 16 == 0 && (uintptr_t)src % 16 == 0)
+      return launch_copy_words(dst, src, n / 4, c->stream);
+    return hipMemcpyAsync(dst, src, n, kind, c->stream);
   }
   int finish() {
     const hipError_t e = hipStreamSynchronize(c->stream);
@@ -877,8 +896,9 @@ extern "C" int hale_matvec(hale_ctx* c, const hale_matrix* m, const float* x, si
   ActBlock* act = (ActBlock*)((char*)s + o2);
   HostStage st(c);
   if ((rc = st.reserve(o2)) || (rc = st.in(dx, x, xlen * 4))) return rc;
-  rc = matvec_enqueue(c, m, dx, dout, act);
-  if (rc || (rc = st.out(out, dout, outlen * 4))) return rc;
+  float* res = st.direct(out, outlen * 4, dout);
+  rc = matvec_enqueue(c, m, dx, res, act);
+  if (rc || (res == dout && (rc = st.out(out, dout, outlen * 4)))) return rc;
   return st.finish();
 }
 
@@ -1050,8 +1070,9 @@ extern "C" int hale_expert_forward(hale_ctx* c, const hale_matrix* gate, const h
   float* dout = (float*)((char*)s + io);
   HostStage st(c);
   if ((rc = st.reserve(2 * io)) || (rc = st.in(dx, x, H * 4))) return rc;
-  rc = expert_enqueue(c, gate, up, down, dx, dout, 2 * io);
-  if (rc || (rc = st.out(out, dout, H * 4))) return rc;
+  float* res = st.direct(out, H * 4, dout);
+  rc = expert_enqueue(c, gate, up, down, dx, res, 2 * io);
+  if (rc || (res == dout && (rc = st.out(out, dout, H * 4)))) return rc;
   return st.finish();
 }
 
