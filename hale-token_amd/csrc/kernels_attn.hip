@@ -586,19 +586,19 @@ constexpr int SMC_ITEMS = (SMC_T * SMC_COLS / 4 + SMC_LOADERS - 1) / SMC_LOADERS
 // exp values in LDS: 4 floats of padding every 32, as in k_rms_norm
 __device__ __host__ constexpr int exp_at(int t) { return t + (t >> 5) * 4; }
 
-// SHORT (rows of at most SMC_THREADS positions, K = 2): the same work-group
-// prepares its head and the new key and scores the head itself, a position
+// SHORT (rows of at most SHORT_MAX positions): the same work-group prepares
+// its head and the new key and scores the head itself, one or two positions
 // per thread, so that a token's attention is one launch; the keys are then
-// read once per head and column block, 1.7 us of L1 reads for 512 positions
-// where the score launch takes 5.  The new position's key and value come
+// read once per head and column block, 1.7 us of L1 reads per 512 positions,
+// where the score launch takes 7.6 us.  The new position's key and value come
 // from the projections: the first work-group of a key/value head pushes them
-// to the cache meanwhile.  Rows up to 190 positions: 9.4 us, where the norm,
-// score and softmax launches took 3.7 + 4.8 + 5.7; up to 512: 10.7 against
-// 15.5.
+// to the cache meanwhile.  Rows up to 190 positions: 8.5 us, where the norm,
+// score and softmax launches took 3.7 + 4.8 + 5.7; up to 512 9.7 against
+// 15.5; from there to 1000 15.0 against 7.6 + 9.8 with a score launch.
+constexpr int SHORT_MAX = 1024;
 template <int K, bool SHORT>  // 256 K >= seq
 __global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(TokenArgs a, const float* __restrict__ scores,
                                                                   int ld, float scale, float* __restrict__ ctx) {
-  static_assert(!SHORT || K == 2, "a position per thread");
   constexpr int T = SMC_T, RP = SMC_RP, NBUF = 3;
   __shared__ __attribute__((aligned(16))) float ebuf[exp_at(256 * K)];
   __shared__ __attribute__((aligned(16))) float prod[NBUF][SMC_COLS * RP];
@@ -652,14 +652,24 @@ __global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(TokenArgs a, c
     if (wave < 2) head.store(a, s_qk + wave * pitch);
     __syncthreads();
     if (c0 == 0 && blockIdx.y == 0 && wave == 6) push_head(a, g, s_qk + pitch);
-    sc[0] = 0.0f;
-    if (wave * 64 < seq - 1) dots.finish(s_qk, pitch, sc);
+#pragma unroll
+    for (int j = 0; j < SPT; j++) {
+      sc[j] = 0.0f;
+      if (SMC_THREADS * j + wave * 64 < seq - 1) {
+        if (j) dots.start(a, g, min(tid + SMC_THREADS * j, seq - 2));
+        dots.finish(s_qk, pitch, &sc[j]);
+      }
+    }
     // the new position, the row's last: by a lane of the last wave, whose
     // own positions few rows reach
     if (tid == SMC_THREADS - 1) red[0] = dot_rows(s_qk, s_qk + pitch, hd);
     __syncthreads();
-    if (tid == seq - 1) sc[0] = red[0];
-    sc[0] = tid < seq ? sc[0] * scale : -INFINITY;
+#pragma unroll
+    for (int j = 0; j < SPT; j++) {
+      const int t = tid + SMC_THREADS * j;
+      if (t == seq - 1) sc[j] = red[0];
+      sc[j] = t < seq ? sc[j] * scale : -INFINITY;
+    }
     __syncthreads();
   } else {
     const float* srow = scores + (size_t)h * ld;
@@ -810,13 +820,13 @@ hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {
   auto softmax_ctx = [&](auto kernel) {
     return launch(kernel, gsc, SMC_THREADS, 0, st, t, (const float*)a.scores, a.ld, scale, a.ctx);
   };
-  if (a.seq <= SMC_THREADS) return softmax_ctx(k_attn_softmax_ctx<2, true>);
+  if (a.seq <= 512) return softmax_ctx(k_attn_softmax_ctx<2, true>);
+  if (a.seq <= SHORT_MAX) return softmax_ctx(k_attn_softmax_ctx<4, true>);
   const dim3 gs((unsigned)((a.seq - 1 + SC_POS - 1) / SC_POS + 1), (unsigned)a.nkv,
                 (unsigned)((group + SC_HEADS - 1) / SC_HEADS));
   hipError_t e = launch(k_attn_scores, gs, 64 * SC_WAVES, (uint32_t)(SC_WAVES * SC_ROWS * (a.hd + 4) * sizeof(float)), st,
                         t, a.ld, scale, a.scores);
   if (e != hipSuccess) return e;
-  if (a.seq <= 1024) return softmax_ctx(k_attn_softmax_ctx<4, false>);
   if (a.seq <= 2048) return softmax_ctx(k_attn_softmax_ctx<8, false>);
   if (a.seq <= 4096) return softmax_ctx(k_attn_softmax_ctx<16, false>);
   if (a.seq <= SMC_MAX) return softmax_ctx(k_attn_softmax_ctx<32, false>);
