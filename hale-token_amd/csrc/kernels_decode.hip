@@ -511,7 +511,6 @@ __global__ __launch_bounds__(64 * RT_E / EM) void k_route_logits_tiled(const flo
                                                                        float* __restrict__ logits,
                                                                        ActBlock* __restrict__ act) {
   constexpr int RT_T = 8 * TM;                           // tokens
-  constexpr int UNROLL = EM > 1 ? 4 : 1;                 // LDS reads ahead of the chains
   constexpr int RT_STRIDE = RT_K + 4;                    // floats per chain row (16-byte aligned)
   constexpr int NT = 64 * RT_E / EM;                     // threads
   constexpr int RT_BUF = (RT_E + RT_T) * 8 * RT_STRIDE;  // floats per buffer
@@ -560,8 +559,7 @@ __global__ __launch_bounds__(64 * RT_E / EM) void k_route_logits_tiled(const flo
     if (c + 1 < nchunk) load_chunk(v, c + 1);  // in flight while chunk c is added
     const float* b = buf[c & 1];
     const int kc = min(RT_K, steps - c * RT_K);  // a multiple of 4 (H % 32 == 0)
-#pragma unroll UNROLL
-    for (int s4 = 0; s4 < kc; s4 += 4) {
+    auto four = [&](int s4) {
       f32x4 wv[EM], xv[TM];
 #pragma unroll
       for (int i = 0; i < EM; i++) wv[i] = *(const f32x4*)(b + wrow + i * 8 * RT_STRIDE + s4);
@@ -573,6 +571,12 @@ __global__ __launch_bounds__(64 * RT_E / EM) void k_route_logits_tiled(const flo
         for (int i = 0; i < EM; i++)
 #pragma unroll
           for (int j = 0; j < TM; j++) acc[i][j] = acc[i][j] + wv[i][q] * xv[j][q];
+    };
+    if constexpr (EM * TM > 1) {
+#pragma unroll 4  // the next reads ahead of the chains
+      for (int s4 = 0; s4 < kc; s4 += 4) four(s4);
+    } else {
+      for (int s4 = 0; s4 < kc; s4 += 4) four(s4);
     }
     if (c + 1 < nchunk) store_chunk(v, buf[(c + 1) & 1]);
     __syncthreads();  // chunk c + 1 staged; every wave is done with chunk c
@@ -2588,23 +2592,26 @@ hipError_t launch_route_logits(const float* router, const float* x, int H, int E
                                ActBlock* act, float* logits, hipStream_t st) {
   if (H > ROUTE_MAX_H || E > ROUTE_MAX_E || H % QK || E < 1 || T < 1) return hipErrorInvalidValue;
   if (T >= ROUTE_TILED_MIN_T) {
-    // many tokens: 16 experts x 8 tokens per work-group, the activation
-    // blocks quantized by the same launch
-    // 16 experts per work-group, or 8 when 16 would leave CUs without one
-    // (Qwen3-30B-A3B layer on the row chains at 48 / 64 / 76 tokens: 103.2-
-    // 103.6 / 112.7-113.2 / 120.3-120.6 -> 101.8-101.9 / 112.3-112.7 /
-    // 118.9-119.3 us per step; Qwen3-235B-A22B at 48: 315-317 -> 310-313)
-    // Register tiles (16 x 16 per work-group of four waves) from 384 of them
-    // on: with one work-group per CU their one wave per SIMD is no faster (500
-    // tokens x 128 experts at H 2048: 24.1 against 21.7 us); 1000 tokens at H
-    // 4096: 73 -> 52 us, 2048 tokens: 131 -> 94 us.
+    // many tokens: tiles of router rows and tokens, the activation blocks
+    // quantized by the same launch.  Eight experts x 8 tokens, a logit per
+    // lane, while tiles of 16 x 16 would leave half the CUs without one
+    // (Qwen3-30B-A3B layer on the row chains at 48 / 64 / 76 tokens, against
+    // 16 experts x 8 tokens: 103.2-103.6 / 112.7-113.2 / 120.3-120.6 ->
+    // 101.8-101.9 / 112.3-112.7 / 118.9-119.3 us per step).  16 x 16 from
+    // 128 of them on, two experts x two tokens per lane (128 experts, H 2048,
+    // 260 / 330 / 500 / 700 tokens: 17.6 / 19.6 / 20.5 / 29.1 us with a logit
+    // per lane, 14.9 / 15.1 / 16.2 / 24.0 so; at 200, 104 tiles, 8 x 8 takes
+    // 10.7); from 384 on four experts x two tokens, which at one work-group
+    // per CU are short of waves (500 tokens 24.1 us): 1000 tokens at H 4096
+    // 73 -> 52 us, 2048 tokens 131 -> 94 us.
     const int tt = (T + 7) / 8, et = (E + 15) / 16, tt16 = (T + 15) / 16;
+    const dim3 grid16(et, tt16);
     if (et * tt16 >= 384)
-      return launch(k_route_logits_tiled<16, 4, 2, 32>, dim3(et, tt16), 256, 0, st, router, x, H, E, T, logits, act);
-    if (et * tt < 256)
-      return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3((E + 7) / 8, tt), 512, 0, st, router, x, H, E, T, logits,
-                    act);
-    return launch(k_route_logits_tiled<16, 1, 1, 64>, dim3(et, tt), 1024, 0, st, router, x, H, E, T, logits, act);
+      return launch(k_route_logits_tiled<16, 4, 2, 32>, grid16, 256, 0, st, router, x, H, E, T, logits, act);
+    if (et * tt16 >= 128)
+      return launch(k_route_logits_tiled<16, 2, 2, 32>, grid16, 512, 0, st, router, x, H, E, T, logits, act);
+    return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3((E + 7) / 8, tt), 512, 0, st, router, x, H, E, T, logits,
+                  act);
   }
   dim3 grid(E, T);
   if (H <= 8 * ROUTE_THREADS)
