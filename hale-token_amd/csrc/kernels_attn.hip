@@ -32,21 +32,22 @@ constexpr int HEAD_MAX = 1024;     // largest head_dim
 //
 // Bound by latency: one load round trip, the ordered sum, one store.  The
 // squares go through LDS to become each lane's K consecutive values
-// (ordered_sum.h); K is the smallest of 4 .. 32 that covers the row, as
-// every unused K costs its predicated loads and chain steps.  One row of
-// 2048: 13.9 us with one chain of squares, 4.5 us so (a launch alone is
-// about 4); the norm and MoE of a Mixtral-shaped layer (rows of 4096) went
-// from 69.4 to 50.4 us.  The sum starts from +0: the reference's -0 start
-// shows only without values.
-template <int K>
-__global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restrict__ delta,
+// (ordered_sum.h); K NT is the smallest that covers the row, as every unused K
+// costs its predicated loads and chain steps.  Rows above 2048 go to 512
+// threads: half as many values per lane, for four more turns of the waves
+// (one row of 4096 / 8192: 6.4 / 9.7 us with 256, 5.5 / 7.3 with 512; 1500 of
+// 8192: 46 and 35).  One row of 2048: 13.9 us with one chain of squares, 4.6
+// so (a launch alone is about 3.5).  The sum starts from +0: the reference's
+// -0 start shows only without values.
+template <int K, int NT>
+__global__ __launch_bounds__(NT) void k_rms_norm(float* x, const float* __restrict__ delta,
                                                   const float* __restrict__ w, int n, float eps,
                                                   float* out) {
   // 4 floats of padding every 32 keep the lanes' 16-byte reads at a stride
   // of K floats off each other's banks
   auto at = [](int i) { return i + (i >> 5) * 4; };
-  __shared__ __attribute__((aligned(16))) float sq[256 * K + 8 * K * 4];
-  __shared__ float part[ordered_lds(4)];
+  __shared__ __attribute__((aligned(16))) float sq[NT * K + NT * K / 8];
+  __shared__ float part[ordered_lds(NT / 64)];
   float* xr = x + (size_t)blockIdx.x * n;
   const float* dr = delta ? delta + (size_t)blockIdx.x * n : nullptr;
   float* orow = out + (size_t)blockIdx.x * n;
@@ -54,7 +55,7 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
   float xv[K], wv[K];
 #pragma unroll
   for (int j = 0; j < K; j++) {
-    const int i = tid + 256 * j;
+    const int i = tid + NT * j;
     if (i < n) {
       xv[j] = xr[i];
       wv[j] = w[i];
@@ -64,12 +65,12 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
     float dv[K];
 #pragma unroll
     for (int j = 0; j < K; j++) {
-      const int i = tid + 256 * j;
+      const int i = tid + NT * j;
       if (i < n) dv[j] = dr[i];
     }
 #pragma unroll
     for (int j = 0; j < K; j++) {
-      const int i = tid + 256 * j;
+      const int i = tid + NT * j;
       if (i < n) {
         xv[j] = xv[j] + dv[j];
         xr[i] = xv[j];
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
   }
 #pragma unroll
   for (int j = 0; j < K; j++) {
-    const int i = tid + 256 * j;
+    const int i = tid + NT * j;
     sq[at(i)] = i < n ? xv[j] * xv[j] : 0.0f;
   }
   __syncthreads();
@@ -92,11 +93,11 @@ __global__ __launch_bounds__(256) void k_rms_norm(float* x, const float* __restr
     v[4 * q + 3] = t.w;
   }
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const float s = team_sum_in_order<K>(v, 0.0f, wave, 4, part);
+  const float s = team_sum_in_order<K>(v, 0.0f, wave, NT / 64, part);
   const float scale = 1.0f / sqrtf(s / (float)n + eps);
 #pragma unroll
   for (int j = 0; j < K; j++) {
-    const int i = tid + 256 * j;
+    const int i = tid + NT * j;
     if (i < n) orow[i] = xv[j] * scale * wv[j];
   }
 }
@@ -799,11 +800,11 @@ hipError_t launch_rms_norm(float* x, const float* delta, const float* w, size_t 
                            float eps, float* out, hipStream_t st) {
   if (rows == 0) return hipSuccess;
   if (n == 0 || n > (size_t)NORM_MAX || rows > 0x7fffffffu) return hipErrorInvalidValue;
-  auto run = [&](auto kernel) { return launch(kernel, (unsigned)rows, 256, 0, st, x, delta, w, (int)n, eps, out); };
-  if (n <= 1024) return run(k_rms_norm<4>);
-  if (n <= 2048) return run(k_rms_norm<8>);
-  if (n <= 4096) return run(k_rms_norm<16>);
-  return run(k_rms_norm<32>);
+  auto run = [&](auto kernel, unsigned nt) { return launch(kernel, (unsigned)rows, nt, 0, st, x, delta, w, (int)n, eps, out); };
+  if (n <= 1024) return run(k_rms_norm<4, 256>, 256);
+  if (n <= 2048) return run(k_rms_norm<8, 256>, 256);
+  if (n <= 4096) return run(k_rms_norm<8, 512>, 512);
+  return run(k_rms_norm<16, 512>, 512);
 }
 
 hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {
