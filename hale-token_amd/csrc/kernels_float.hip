@@ -27,7 +27,6 @@ namespace hale {
 
 constexpr int FR = 8;        // rows per work-group (FR * 8 fold threads, whole waves)
 constexpr int FK = 512;      // columns per chunk
-constexpr int NS = 4;        // chunks in flight
 constexpr int FPAD = 8;      // row pitch FK + FPAD = 8 (mod 64) floats: the fold
                              // threads (row r, chain l) of a wave read banks 8r + l
 
@@ -75,8 +74,9 @@ struct FloatMats {
 
 // VEC: every row starts 16-byte aligned, so a piece is one 16-byte load;
 // otherwise it is read value by value.  MANY: several matrices; one alone
-// skips the choice (2 % of a 151,936 x 2048 projection's time).
-template <int DT, bool VEC, bool MANY>
+// skips the choice (2 % of a 151,936 x 2048 projection's time).  NS: chunks
+// in flight (float_ring).
+template <int DT, bool VEC, bool MANY, int NS>
 __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __restrict__ x,
                                                     int cols) {
   constexpr int PER = FloatFmt<DT>::PER16;
@@ -105,11 +105,14 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
     float x[PER];
   };
   auto load = [&](Regs& R, int ch) {
-    // `done` is a multiple of 8 and PER 4 or 8: pieces past the row's end
-    // repeat the last one, rows past the matrix's the last (loaded, never
-    // written; every load unconditional, so that several chunks stay in
-    // flight)
-    const int c = min(ch * FK + cpiece, done - PER);
+    // `done` is a multiple of 8 and PER 4 or 8, so a piece below `done` ends
+    // at or before it; rows past the matrix's end are clamped (loaded, never
+    // written).  With several chunks in flight pieces past the row's end repeat
+    // the last one: every load is then unconditional, where under a branch
+    // each would wait for the one before.
+    const int cp = ch * FK + cpiece;
+    if (NS == 1 && cp >= done) return;
+    const int c = NS == 1 ? cp : min(cp, done - PER);
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
       const int r = min(row0 + j * RPP + tid / UPR, rows - 1);
@@ -158,11 +161,11 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
     if (next >= 0) load(R, next);
     if (tid < NF) acc = lds_sum_strided<8>(&P[fr][fl], ncols / 8, acc);
   };
-  // NS chunks in flight where a row has as many: one round trip for a row of
-  // 2048 instead of four
+  // NS chunks in flight (the launcher's rows have as many): one round trip
+  // for a bf16 row of 2048 instead of four
   Regs R[NS];
   int ch = 0;
-  if (nchunks >= NS) {
+  if constexpr (NS > 1) {
 #pragma unroll
     for (int j = 0; j < NS; j++) {
       load(R[j], j);
@@ -279,6 +282,20 @@ hipError_t launch_encode_half(int dtype, const float* values, size_t n, void* ou
                       : launch(k_encode_half<BF16>, grid, 256, 0, st, values, n, o);
 }
 
+// Chunks in flight.  Several where waits for the round trip show: with fewer
+// than two work-groups per CU (cold, one chunk / several: bf16 512 x 2048 5.1 /
+// 4.8 us, 2048 x 4096 8.7 / 8.1, 3000 x 14336 28.9 / 25.8, f32 2048 x 2048 6.8 /
+// 6.1), and for half rows of exactly four chunks, which one pass of straight
+// code covers (5120 x 2048 8.1 / 7.4, 151,936 x 2048 102 / 97.6).  With more
+// work-groups they cover for each other, and the longer code and its registers
+// cost (bf16 4096 x 4096 10.1 / 10.7, f32 40,000 x 1500 40.4 / 42.0).
+static int float_ring(int dtype, size_t cols, size_t groups) {
+  const size_t nchunks = (cols / 8 * 8 + FK - 1) / FK;
+  const int ns = dtype == F32 ? 2 : 4;
+  if (nchunks < (size_t)ns) return 1;
+  return groups < 512 || (dtype != F32 && nchunks == 4) ? ns : 1;
+}
+
 hipError_t launch_gemv_float(int dtype, const void* w, const float* x, size_t rows, size_t cols,
                              float* out, hipStream_t st) {
   return launch_gemv_float_many(dtype, 1, &w, x, &rows, cols, &out, st);
@@ -305,13 +322,16 @@ hipError_t launch_gemv_float_many(int dtype, int n, const void* const* w, const 
   }
   if (groups == 0) return hipSuccess;
   auto run = [&](auto kernel) { return launch(kernel, (unsigned)groups, 256, 0, st, m, x, (int)cols); };
-#define HALE_FLOAT_CASE(D)                                                        \
-  if (dtype == D)                                                                 \
-    return vec ? (n > 1 ? run(k_gemv_float<D, true, true>) : run(k_gemv_float<D, true, false>)) \
-               : (n > 1 ? run(k_gemv_float<D, false, true>) : run(k_gemv_float<D, false, false>));
+  const bool ring = float_ring(dtype, cols, groups) > 1;
+#define HALE_FLOAT_RING(D, V, M) (ring ? run(k_gemv_float<D, V, M, D == F32 ? 2 : 4>) : run(k_gemv_float<D, V, M, 1>))
+#define HALE_FLOAT_CASE(D)                                                                      \
+  if (dtype == D)                                                                               \
+    return vec ? (n > 1 ? HALE_FLOAT_RING(D, true, true) : HALE_FLOAT_RING(D, true, false))     \
+               : (n > 1 ? HALE_FLOAT_RING(D, false, true) : HALE_FLOAT_RING(D, false, false));
   HALE_FLOAT_CASE(F32)
   HALE_FLOAT_CASE(F16)
   HALE_FLOAT_CASE(BF16)
+#undef HALE_FLOAT_RING
 #undef HALE_FLOAT_CASE
   return hipErrorInvalidValue;
 }
