@@ -116,6 +116,10 @@ def build(ctx, dtype, Hd, nh, nkv, hd, seed, qk_norm, max_len):
     qn = kn = None
     if qk_norm:
         qn, kn = O.normal(seed + 10, hd, 1.0, 0.1), O.normal(seed + 11, hd, 1.0, 0.1)
+    if qk_norm == "q":
+        kn = None
+    if qk_norm == "k":
+        qn = None
     ref = O.OracleAttention(dtype, Hd, nh, nkv, hd, 1e-6, *mats, q_norm=qn, k_norm=kn, max_len=max_len)
     att = H.Attention(ctx, *gm, qn, kn, nh, nkv, hd, 1e-6, max_len=max_len)
     return ref, att
@@ -154,6 +158,23 @@ def test_attention_projections_together(ctx, dtype, Hd, nh, nkv, hd):
         x = O.normal(700 + pos, Hd)
         c, s = O.rope_angles(hd, 1e6, pos)
         assert same_bits(att.forward(x, pos, c, s), ref.forward(x, c, s)), pos
+    att.close()
+
+
+@pytest.mark.parametrize("norms", ["q", "k", ""])
+@pytest.mark.parametrize("hd", [128, 144])
+def test_attention_one_sided_norms(ctx, norms, hd):
+    # only the queries normed, only the keys, or neither (then no wave sums
+    # squares), in the one launch for short rows and in the score kernel for
+    # longer ones; heads of one register pass and with a remainder of 16
+    ref, att = build(ctx, O.F32, 64, 3, 1, hd, seed=hd, qk_norm=norms, max_len=1030)
+    for pos in range(1030):
+        x = O.normal(7000 + pos, 64, 0.0, 3.0)
+        c, s = O.rope_angles(hd, 1e6, pos)
+        got = att.forward(x, pos, c, s)
+        want = ref.forward(x, c, s)
+        if pos < 4 or pos % 200 == 0 or pos >= 1022:
+            assert same_bits(got, want), pos
     att.close()
 
 
