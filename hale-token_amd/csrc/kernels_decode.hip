@@ -489,9 +489,10 @@ __global__ __launch_bounds__(ROUTE_THREADS) void k_route_logits(const float* __r
 // chunks of RT_K steps, two buffers, so chunk c + 1 loads while chunk c is added,
 // and every staged row serves 8 TM or RT_E logits.  The two rounded operations
 // per product bound it; with one logit per lane (EM = TM = 1) every four of
-// them wait for two 16-byte LDS reads, and the reads bound it instead.  Four
-// experts and two tokens per lane read six times per 32 products: 2048 tokens
-// x 128 experts at H 4096 131 -> 94 us.  The eight chains of a logit
+// them wait for two 16-byte LDS reads, and the reads bound it instead.  Two
+// experts and two tokens per lane read four times per 16 products: 2048 tokens
+// x 128 experts at H 4096 124 -> 80 us (four experts x two tokens, with half the
+// waves, 90: nowhere the fastest).  The eight chains of a logit
 // are reduced in the one-token kernel's fixed order, so each logit has its
 // bits.  Then the work-groups quantize the token tile's activation blocks
 // (as k_act_quant does), each taking its share: block q of the tile goes to
@@ -598,7 +599,7 @@ __global__ __launch_bounds__(64 * RT_E / EM) void k_route_logits_tiled(const flo
       }
     }
   // this work-group's share of the tile's activation blocks, 8 lanes per
-  // block, 128 blocks per pass (the bound is uniform per 8-lane group)
+  // block, NT / 8 blocks per pass (the bound is uniform per 8-lane group)
   const int nb = H / QK;
   const int nq = min(RT_T, T - t0) * nb;
   for (int q = blockIdx.x + gridDim.x * (tid >> 3); q < nq; q += gridDim.x * (NT / 8)) {
@@ -2594,24 +2595,22 @@ hipError_t launch_route_logits(const float* router, const float* x, int H, int E
   if (T >= ROUTE_TILED_MIN_T) {
     // many tokens: tiles of router rows and tokens, the activation blocks
     // quantized by the same launch.  Eight experts x 8 tokens, a logit per
-    // lane, while tiles of 16 x 16 would leave half the CUs without one
-    // (Qwen3-30B-A3B layer on the row chains at 48 / 64 / 76 tokens, against
-    // 16 experts x 8 tokens: 103.2-103.6 / 112.7-113.2 / 120.3-120.6 ->
-    // 101.8-101.9 / 112.3-112.7 / 118.9-119.3 us per step).  16 x 16 from
-    // 128 of them on, two experts x two tokens per lane (128 experts, H 2048,
-    // 260 / 330 / 500 / 700 tokens: 17.6 / 19.6 / 20.5 / 29.1 us with a logit
-    // per lane, 14.9 / 15.1 / 16.2 / 24.0 so; at 200, 104 tiles, 8 x 8 takes
-    // 10.7); from 384 on four experts x two tokens, which at one work-group
-    // per CU are short of waves (500 tokens 24.1 us): 1000 tokens at H 4096
-    // 73 -> 52 us, 2048 tokens 131 -> 94 us.
-    const int tt = (T + 7) / 8, et = (E + 15) / 16, tt16 = (T + 15) / 16;
-    const dim3 grid16(et, tt16);
-    if (et * tt16 >= 384)
-      return launch(k_route_logits_tiled<16, 4, 2, 32>, grid16, 256, 0, st, router, x, H, E, T, logits, act);
-    if (et * tt16 >= 128)
-      return launch(k_route_logits_tiled<16, 2, 2, 32>, grid16, 512, 0, st, router, x, H, E, T, logits, act);
-    return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3((E + 7) / 8, tt), 512, 0, st, router, x, H, E, T, logits,
-                  act);
+    // lane, while two of them per CU (what their LDS allows) take the whole
+    // call at once: 128 experts, 256 tokens (512 work-groups) 13.1 us at H
+    // 2048 and 19.7 at H 4096, with 16 x 16 tiles 16.8 and 27.5; 257 tokens
+    // 18.8 and 29.8 against 17.1 and 27.6, 600 tokens 26.1 and 43.5 against
+    // 23.8 and 39.4.  16 x 16 beyond, two experts x two tokens per lane (2048
+    // tokens x 128 experts 44.0 and 80.2 us, 68.3 and 124 with 8 x 8), but
+    // 8 x 8 at any length for up to 8 experts, of whose 16-row tile half is
+    // padding (H 4096, 2056 / 4096 / 8192 tokens: 34.3 / 39.6 / 75.3 us
+    // against 48.4 / 52.4 / 79.6), and for up to 32 experts until 16 x 16 tiles
+    // come to three quarters of the CUs (H 4096, 16 experts x 2056 / 3000 / 4096
+    // tokens, 129 / 188 / 256 tiles: 41.3 / 45.0 / 55.4 against 48.6 / 49.3 /
+    // 52.8; 64 experts draw there).
+    const int et8 = (E + 7) / 8, tt8 = (T + 7) / 8, et = (E + 15) / 16, tt = (T + 15) / 16;
+    if ((size_t)et8 * tt8 <= 512 || (E <= 8 && tt8 <= 0xffff) || (E <= 32 && et * tt < 192))
+      return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3(et8, tt8), 512, 0, st, router, x, H, E, T, logits, act);
+    return launch(k_route_logits_tiled<16, 2, 2, 32>, dim3(et, tt), 512, 0, st, router, x, H, E, T, logits, act);
   }
   dim3 grid(E, T);
   if (H <= 8 * ROUTE_THREADS)
