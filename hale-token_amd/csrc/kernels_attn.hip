@@ -135,7 +135,9 @@ __device__ __forceinline__ void wave_lds_sync() {
 // squares is one chain per head, a lane each; a wave none of whose heads is
 // normed skips it (without QK-norm, 1100 positions of 32 heads of 128: 27.1 ->
 // 25.6 us a token; 190 of 16 heads of 256 23.6 -> 21.7, of 4 heads of 1024 44.8
-// -> 37.0).
+// -> 37.0).  Beyond 128 values the heads' loads go out side by side (8 heads of
+// 1024 with QK-norm, 520 positions by two launches: 75.5 us a head after the
+// other, 66.1 so).
 template <int R>
 struct HeadRows {
   const float* src[R];   // wave-uniform
@@ -156,12 +158,14 @@ struct HeadRows {
   __device__ __forceinline__ void store(const TokenArgs& a, float* rows) {
     const int lane = __lane_id(), hd = a.hd, half = hd / 2, pitch = hd + 4;
 #pragma unroll
-    for (int r = 0; r < R; r++) {
+    for (int r = 0; r < R; r++)
 #pragma unroll
       for (int j = 0; j < 2; j++)
         if (lane + 64 * j < hd) rows[r * pitch + lane + 64 * j] = x[r][j];
-      for (int c = 128 + lane; c < hd; c += 64) rows[r * pitch + c] = src[r][c];
-    }
+#pragma unroll 4
+    for (int c = 128 + lane; c < hd; c += 64)
+#pragma unroll
+      for (int r = 0; r < R; r++) rows[r * pitch + c] = src[r][c];
     wave_lds_sync();
     float scale = 0.0f;  // inverse_rms (src/ops/norm.rs:25-28), in order from -0.0
     bool any = false;    // uniform
@@ -183,23 +187,31 @@ struct HeadRows {
       }
       wave_lds_sync();
     }
+    // rms_norm_in_place: x = x * (scale * w)
+    float sc[R];
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      const float sc = lane_value(scale, r);
-      const bool normed = norm[r] != nullptr;
-      float* row = rows + r * pitch;
-      // rms_norm_in_place: x = x * (scale * w)
-      if (hd <= 128) {
+    for (int r = 0; r < R; r++) sc[r] = lane_value(scale, r);
+    if (hd <= 128) {
+#pragma unroll
+      for (int r = 0; r < R; r++)
 #pragma unroll
         for (int j = 0; j < 2; j++)
-          if (lane + 64 * j < hd) row[lane + 64 * j] = normed ? x[r][j] * (sc * w[r][j]) : x[r][j];
-      } else if (normed) {
-        for (int c = lane; c < hd; c += 64) row[c] = row[c] * (sc * norm[r][c]);
-      }
-      wave_lds_sync();
-      for (int c = lane; c < half; c += 64) {  // Rope::apply (src/ops/rope.rs:36-44)
+          if (norm[r] && lane + 64 * j < hd) rows[r * pitch + lane + 64 * j] = x[r][j] * (sc[r] * w[r][j]);
+    } else if (any) {
+#pragma unroll 4
+      for (int c = lane; c < hd; c += 64)
+#pragma unroll
+        for (int r = 0; r < R; r++)
+          if (norm[r]) rows[r * pitch + c] = rows[r * pitch + c] * (sc[r] * norm[r][c]);
+    }
+    wave_lds_sync();
+#pragma unroll 2
+    for (int c = lane; c < half; c += 64) {  // Rope::apply (src/ops/rope.rs:36-44)
+      const float cc = c < 64 ? cs : a.cos[c], ss = c < 64 ? sn : a.sin[c];
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        float* row = rows + r * pitch;
         const float p = row[c], q = row[half + c];
-        const float cc = c < 64 ? cs : a.cos[c], ss = c < 64 ? sn : a.sin[c];
         row[c] = p * cc - q * ss;
         row[half + c] = q * cc + p * ss;
       }

@@ -180,11 +180,11 @@ def test_attention_one_sided_norms(ctx, norms, hd):
 
 @pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 32), (16, 2, 16), (16, 1, 16), (6, 2, 16), (4, 4, 16)])
 def test_attention_long_context(ctx, nh, nkv, hd):
-    # 1100 positions with GQA groups of 4, 8, 16, 3 and 1: 35 score blocks of
-    # 32 positions, three softmax pipeline steps of 512, and context passes
-    # over five 256-position tiles, so a register stage of the value stream
-    # is refilled and both LDS buffers alternate; groups 3 and 1 leave a
-    # work-group of the softmax + context kernel with one query head
+    # 1100 positions with GQA groups of 4, 8, 16, 3 and 1: rows of one launch,
+    # then 18 score blocks of 64 positions and context passes over nine
+    # 128-position tiles, so every register stage of the value stream is
+    # refilled and the three LDS buffers alternate; group 16 takes two score
+    # work-groups, groups 3 and 1 leave a score wave with one query head
     ref, att = build(ctx, O.BF16, 256, nh, nkv, hd, seed=77, qk_norm=True, max_len=1100)
     for pos in range(1100):
         x = O.normal(5000 + pos, 256)
@@ -196,11 +196,29 @@ def test_attention_long_context(ctx, nh, nkv, hd):
     att.close()
 
 
+@pytest.mark.parametrize("nh,nkv,hd,qk,steps", [
+    (8, 1, 128, True, 1100),   # past 1024 positions two key chunks per score wave
+    (3, 1, 272, True, 1100),   # both key register sets refilled, two or three heads per wave
+    (9, 1, 1024, True, 140),
+])
+def test_attention_wide_heads(ctx, nh, nkv, hd, qk, steps):
+    ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=nh + hd, qk_norm=qk, max_len=steps)
+    edges = {n - 1 for c in (1, 64, 128, 512, 768, 1024, 1088) for n in (c, c + 1, c + 2)}
+    for pos in range(steps):
+        x = O.normal(3000 + pos, 64, 0.0, 3.0)
+        c, s = O.rope_angles(hd, 1e6, pos)
+        got = att.forward(x, pos, c, s)
+        want = ref.forward(x, c, s)
+        if pos in edges or pos == steps - 1:
+            assert same_bits(got, want), pos
+    att.close()
+
+
 @pytest.mark.parametrize("nh,nkv,hd,steps", [(2, 1, 80, 2060), (3, 1, 272, 600), (2, 2, 16, 4100)])
 def test_attention_softmax_context_edges(ctx, nh, nkv, hd, steps):
     # both sides of the row lengths that pick the values per lane of the
     # ordered sum, of the 128-position tiles and of their 64-position batches,
-    # and of the rows that one launch takes (512), with head sizes whose last
+    # and of the rows that one launch takes (512, 1024), with head sizes whose last
     # column block is half full and whose keys fill several chunks of 64
     ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=hd, qk_norm=True, max_len=steps)
     edges = {n - 1 for c in (1, 32, 64, 128, 192, 256, 384, 512, 1024, 2048, 4096) for n in (c, c + 1, c + 2)}
