@@ -607,16 +607,26 @@ constexpr int SMC_ITEMS = (SMC_T * SMC_COLS / 4 + SMC_LOADERS - 1) / SMC_LOADERS
 // exp values in LDS: 4 floats of padding every 32, as in k_rms_norm
 __device__ __host__ constexpr int exp_at(int t) { return t + (t >> 5) * 4; }
 
-// SHORT (rows of at most SHORT_MAX positions): the same work-group prepares
-// its head and the new key and scores the head itself, one or two positions
-// per thread, so that a token's attention is one launch; the keys are then
-// read once per head and column block, 1.7 us of L1 reads per 512 positions,
-// where the score launch takes 7.6 us.  The new position's key and value come
-// from the projections: the first work-group of a key/value head pushes them
-// to the cache meanwhile.  Rows up to 190 positions: 8.5 us, where the norm,
-// score and softmax launches took 3.7 + 4.8 + 5.7; up to 512 9.7 against
-// 15.5; from there to 1000 15.0 against 7.6 + 9.8 with a score launch.
-constexpr int SHORT_MAX = 1024;
+// SHORT: the same work-group prepares its head and the new key and scores the
+// head itself, one or two positions per thread, so that a token's attention is
+// one launch.  The new position's key and value come from the projections: the
+// first work-group of a key/value head pushes them to the cache meanwhile.
+// Against it stand the scores, formed once per column block: the longer the
+// row and the larger the head, the more keys each work-group reads through L1.
+// Its registers admit one work-group per CU, so beyond 256 of them it runs in
+// turns.  Hence at most SHORT_GROUPS work-groups, and rows up to 512; to 768
+// where a norm, which the score launch would do in front of its keys, lengthens
+// the other way, and the head has at most SHORT_HEAD values.  A token's whole
+// call, one launch / two, us: 32 heads of 128, QK-norm, four key/value heads,
+// 190 / 440 / 520 / 760 / 900 positions 19.4 / 21.8 / 23.1 / 25.4 / 26.5 and
+// 23.2 / 24.6 / 25.1 / 26.1 / 26.6; without the norm 19.1 / 21.6 / 22.9 / 25.1 /
+// 26.1 and 20.9 / 22.4 / 22.9 / 24.0 / 24.5; 64 heads (256 work-groups) 520
+// positions 29.2 / 30.9; 96 heads (384) 190 positions 39.2 / 35.7; 16 heads of
+// 256, 440 / 520 positions 27.9 / 30.0 and 28.5 / 29.1; 16 heads of 512, 190 /
+// 520 positions 36.9 / 50.5 and 41.8 / 44.3.
+constexpr int SHORT_MAX = 768;
+constexpr int SHORT_HEAD = 128;
+constexpr unsigned SHORT_GROUPS = 256;
 template <int K, bool SHORT>  // 256 K >= seq
 __global__ __launch_bounds__(SMC_THREADS) void k_attn_softmax_ctx(TokenArgs a, const float* __restrict__ scores,
                                                                   int ld, float scale, float* __restrict__ ctx) {
@@ -841,8 +851,11 @@ hipError_t launch_attention_core(const AttnArgs& a, hipStream_t st) {
   auto softmax_ctx = [&](auto kernel) {
     return launch(kernel, gsc, SMC_THREADS, 0, st, t, (const float*)a.scores, a.ld, scale, a.ctx);
   };
-  if (a.seq <= 512) return softmax_ctx(k_attn_softmax_ctx<2, true>);
-  if (a.seq <= SHORT_MAX) return softmax_ctx(k_attn_softmax_ctx<4, true>);
+  const bool normed = a.q_norm || a.k_norm;
+  if (gsc.x * gsc.y <= SHORT_GROUPS && a.seq <= (normed && a.hd <= SHORT_HEAD ? SHORT_MAX : 512)) {
+    if (a.seq <= 512) return softmax_ctx(k_attn_softmax_ctx<2, true>);
+    return softmax_ctx(k_attn_softmax_ctx<4, true>);
+  }
   const dim3 gs((unsigned)((a.seq - 1 + SC_POS - 1) / SC_POS + 1), (unsigned)a.nkv,
                 (unsigned)((group + SC_HEADS - 1) / SC_HEADS));
   hipError_t e = launch(k_attn_scores, gs, 64 * SC_WAVES, (uint32_t)(SC_WAVES * SC_ROWS * (a.hd + 4) * sizeof(float)), st,

@@ -197,11 +197,15 @@ def test_attention_long_context(ctx, nh, nkv, hd):
 
 
 @pytest.mark.parametrize("nh,nkv,hd,qk,steps", [
-    (8, 1, 128, True, 1100),   # past 1024 positions two key chunks per score wave
-    (3, 1, 272, True, 1100),   # both key register sets refilled, two or three heads per wave
-    (9, 1, 1024, True, 140),
+    (8, 1, 128, True, 1100),   # one launch to 768 positions, then two key chunks per score wave
+    (8, 1, 128, False, 520),   # one launch to 512
+    (3, 1, 272, True, 1100),   # one launch to 512, then both key register sets refilled
+    (5, 5, 144, True, 800),
+    (8, 2, 1024, True, 520),   # 256 work-groups
+    (9, 1, 1024, True, 140),   # 288: scores and context in two launches from the first position
+    (16, 2, 528, False, 70),   # 272, heads whose last column block is half full
 ])
-def test_attention_wide_heads(ctx, nh, nkv, hd, qk, steps):
+def test_attention_one_or_two_launches(ctx, nh, nkv, hd, qk, steps):
     ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=nh + hd, qk_norm=qk, max_len=steps)
     edges = {n - 1 for c in (1, 64, 128, 512, 768, 1024, 1088) for n in (c, c + 1, c + 2)}
     for pos in range(steps):
@@ -218,7 +222,7 @@ def test_attention_wide_heads(ctx, nh, nkv, hd, qk, steps):
 def test_attention_softmax_context_edges(ctx, nh, nkv, hd, steps):
     # both sides of the row lengths that pick the values per lane of the
     # ordered sum, of the 128-position tiles and of their 64-position batches,
-    # and of the rows that one launch takes (512, 1024), with head sizes whose last
+    # and of the rows that one launch takes (512, 768), with head sizes whose last
     # column block is half full and whose keys fill several chunks of 64
     ref, att = build(ctx, O.F32, 64, nh, nkv, hd, seed=hd, qk_norm=True, max_len=steps)
     edges = {n - 1 for c in (1, 32, 64, 128, 192, 256, 384, 512, 1024, 2048, 4096) for n in (c, c + 1, c + 2)}
