@@ -15,9 +15,8 @@
 // converts f16/bf16 to f32, and parks the products in LDS; wave 0 then folds
 // them, lane (row r, chain l) reading products 8i + l of row r in order.
 // Two LDS buffers; the loads of up to NS chunks are in flight during a fold.
-// HBM-bound for many rows (151,936 x 2048 bf16: 102-103 us with one chunk in
-// flight, 97.6 us with four: 6.4 TB/s); few rows wait for the round trip and
-// wave 0's fold (5120 x 2048 bf16 8.1 -> 7.4 us).
+// HBM-bound for many rows (151,936 x 2048 bf16, not in the caches: 110 us, 5.7
+// TB/s); few rows wait for the round trips and wave 0's fold.
 #pragma clang fp contract(off)
 
 #include "hale_device.h"
@@ -58,27 +57,12 @@ __device__ __forceinline__ void unpack16(const u32x4& v, float* o) {
   }
 }
 
-// The matrices of one launch (all cols long): work-groups first[i] ..
-// first[i + 1] - 1 take matrix i.
-struct FloatMats {
-  const uint8_t* w[MATVEC_MANY];
-  float* out[MATVEC_MANY];
-  int rows[MATVEC_MANY], first[MATVEC_MANY];
-  __device__ __forceinline__ int of(int group) const {
-    int i = 0;
-#pragma unroll
-    for (int j = 1; j < MATVEC_MANY; j++) i = group >= first[j] ? j : i;
-    return i;
-  }
-};
-
-// VEC: every row starts 16-byte aligned, so a piece is one 16-byte load;
-// otherwise it is read value by value.  MANY: several matrices; one alone
-// skips the choice (2 % of a 151,936 x 2048 projection's time).  NS: chunks
-// in flight (float_ring).
-template <int DT, bool VEC, bool MANY, int NS>
-__global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __restrict__ x,
-                                                    int cols) {
+// Rows row0 .. row0 + FR - 1 of one matrix, by one work-group.  VEC: every row
+// starts 16-byte aligned, so a piece is one 16-byte load; otherwise it is read
+// value by value.  NS: chunks in flight (float_ring).
+template <int DT, bool VEC, int NS>
+__device__ __forceinline__ void gemv_float_rows(const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                int row0, int rows, int cols, float* __restrict__ out) {
   constexpr int PER = FloatFmt<DT>::PER16;
   constexpr int ESZ = DT == F32 ? 4 : 2;
   constexpr int UPR = FK / PER;          // 16-byte pieces per row of a chunk
@@ -89,11 +73,6 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
   __shared__ __attribute__((aligned(16))) float prod[2][FR][FK + FPAD];
 
   const int tid = threadIdx.x;
-  const int mi = MANY ? m.of((int)blockIdx.x) : 0;
-  const uint8_t* __restrict__ w = m.w[mi];
-  float* __restrict__ out = m.out[mi];
-  const int rows = m.rows[mi];
-  const int row0 = ((int)blockIdx.x - m.first[mi]) * FR;
   const int done = cols / 8 * 8;         // columns covered by the lane accumulators
   const int nchunks = (done + FK - 1) / FK;
   const size_t rb = (size_t)cols * ESZ;  // row bytes
@@ -111,30 +90,34 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
     // the last one: every load is then unconditional, where under a branch
     // each would wait for the one before.
     const int cp = ch * FK + cpiece;
-    if (NS == 1 && cp >= done) return;
     const int c = NS == 1 ? cp : min(cp, done - PER);
+    const bool in = NS > 1 || c < done;
 #pragma unroll
     for (int j = 0; j < LPT; j++) {
       const int r = min(row0 + j * RPP + tid / UPR, rows - 1);
       const uint8_t* src = w + (size_t)r * rb + (size_t)c * ESZ;
-      if constexpr (VEC) {
-        R.w[j] = __builtin_nontemporal_load((const u32x4*)src);
-      } else if constexpr (DT == F32) {
-        const unsigned* s4 = (const unsigned*)src;
-        R.w[j] = u32x4{s4[0], s4[1], s4[2], s4[3]};
-      } else {
-        const uint16_t* s2 = (const uint16_t*)src;
-        R.w[j] = u32x4{s2[0] | ((unsigned)s2[1] << 16), s2[2] | ((unsigned)s2[3] << 16),
-                       s2[4] | ((unsigned)s2[5] << 16), s2[6] | ((unsigned)s2[7] << 16)};
+      if (in) {
+        if constexpr (VEC) {
+          R.w[j] = __builtin_nontemporal_load((const u32x4*)src);
+        } else if constexpr (DT == F32) {
+          const unsigned* s4 = (const unsigned*)src;
+          R.w[j] = u32x4{s4[0], s4[1], s4[2], s4[3]};
+        } else {
+          const uint16_t* s2 = (const uint16_t*)src;
+          R.w[j] = u32x4{s2[0] | ((unsigned)s2[1] << 16), s2[2] | ((unsigned)s2[3] << 16),
+                         s2[4] | ((unsigned)s2[5] << 16), s2[6] | ((unsigned)s2[7] << 16)};
+        }
       }
     }
+    if (in) {
 #pragma unroll
-    for (int q = 0; q < PER / 4; q++) {
-      const f32x4 v = *(const f32x4*)(x + c + 4 * q);
-      R.x[4 * q] = v.x;
-      R.x[4 * q + 1] = v.y;
-      R.x[4 * q + 2] = v.z;
-      R.x[4 * q + 3] = v.w;
+      for (int q = 0; q < PER / 4; q++) {
+        const f32x4 v = *(const f32x4*)(x + c + 4 * q);
+        R.x[4 * q] = v.x;
+        R.x[4 * q + 1] = v.y;
+        R.x[4 * q + 2] = v.z;
+        R.x[4 * q + 3] = v.w;
+      }
     }
   };
 
@@ -142,8 +125,8 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
   constexpr int NF = FR * 8;
   const int fr = tid >> 3, fl = tid & 7;
   float acc = 0.0f;
-  // chunk ch from R, which then takes chunk `next` (none: negative)
-  auto step = [&](Regs& R, int ch, int next) {
+  // chunk ch from R, which then takes chunk `next` if there is one
+  auto step = [&](Regs& R, int ch, int next, bool more) {
     const int c0 = ch * FK;
     const int ncols = min(FK, done - c0);
     float(*P)[FK + FPAD] = prod[ch & 1];
@@ -158,14 +141,13 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
       }
     }
     __syncthreads();
-    if (next >= 0) load(R, next);
+    if (more) load(R, next);
     if (tid < NF) acc = lds_sum_strided<8>(&P[fr][fl], ncols / 8, acc);
   };
-  // NS chunks in flight (the launcher's rows have as many): one round trip
-  // for a bf16 row of 2048 instead of four
+  // NS chunks in flight (the launcher's rows have as many)
   Regs R[NS];
-  int ch = 0;
   if constexpr (NS > 1) {
+    int ch = 0;
 #pragma unroll
     for (int j = 0; j < NS; j++) {
       load(R[j], j);
@@ -173,16 +155,16 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
     }
     for (; ch + 2 * NS <= nchunks; ch += NS)
 #pragma unroll
-      for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j);
+      for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j, true);
 #pragma unroll
-    for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j < nchunks ? ch + NS + j : -1);
+    for (int j = 0; j < NS; j++) step(R[j], ch + j, ch + NS + j, ch + NS + j < nchunks);
     ch += NS;
 #pragma unroll
     for (int j = 0; j < NS; j++)
-      if (ch + j < nchunks) step(R[j], ch + j, -1);
-  } else if (nchunks > 0) {
-    load(R[0], 0);
-    for (; ch < nchunks; ch++) step(R[0], ch, ch + 1 < nchunks ? ch + 1 : -1);
+      if (ch + j < nchunks) step(R[j], ch + j, 0, false);
+  } else {
+    if (nchunks > 0) load(R[0], 0);
+    for (int ch = 0; ch < nchunks; ch++) step(R[0], ch, ch + 1, ch + 1 < nchunks);
   }
 
   if (tid < NF) {
@@ -213,6 +195,29 @@ __global__ __launch_bounds__(256) void k_gemv_float(FloatMats m, const float* __
       out[row] = red + tail;
     }
   }
+}
+
+template <int DT, bool VEC, int NS>
+__global__ __launch_bounds__(256) void k_gemv_float(const uint8_t* __restrict__ w, const float* __restrict__ x,
+                                                    int rows, int cols, float* __restrict__ out) {
+  gemv_float_rows<DT, VEC, NS>(w, x, blockIdx.x * FR, rows, cols, out);
+}
+
+// The matrices of one launch (all cols long): work-groups first[i] ..
+// first[i + 1] - 1 take matrix i.
+struct FloatMats {
+  const uint8_t* w[MATVEC_MANY];
+  float* out[MATVEC_MANY];
+  int rows[MATVEC_MANY], first[MATVEC_MANY];
+};
+
+template <int DT, bool VEC, int NS>
+__global__ __launch_bounds__(256) void k_gemv_float_many(FloatMats m, const float* __restrict__ x, int cols) {
+  const int g = blockIdx.x;
+  int i = 0;
+#pragma unroll
+  for (int j = 1; j < MATVEC_MANY; j++) i = g >= m.first[j] ? j : i;
+  gemv_float_rows<DT, VEC, NS>(m.w[i], x, (g - m.first[i]) * FR, m.rows[i], cols, m.out[i]);
 }
 
 // encode_row for the half formats (src/tensor/quant.rs:274-292): half's
@@ -282,23 +287,50 @@ hipError_t launch_encode_half(int dtype, const float* values, size_t n, void* ou
                       : launch(k_encode_half<BF16>, grid, 256, 0, st, values, n, o);
 }
 
-// Chunks in flight.  Several where waits for the round trip show: with fewer
-// than two work-groups per CU (cold, one chunk / several: bf16 512 x 2048 5.1 /
-// 4.8 us, 2048 x 4096 8.7 / 8.1, 3000 x 14336 28.9 / 25.8, f32 2048 x 2048 6.8 /
-// 6.1), and for half rows of exactly four chunks, which one pass of straight
-// code covers (5120 x 2048 8.1 / 7.4, 151,936 x 2048 102 / 97.6).  With more
-// work-groups they cover for each other, and the longer code and its registers
-// cost (bf16 4096 x 4096 10.1 / 10.7, f32 40,000 x 1500 40.4 / 42.0).
-static int float_ring(int dtype, size_t cols, size_t groups) {
+// Whether a launch keeps several chunks in flight (two of f32, four of half
+// values) instead of one ahead: rows of four chunks and more, and either at most
+// a work-group per CU, where nothing else covers the round trips, or half rows so
+// many that the launch is a stream through memory.  Between them a CU's
+// work-groups cover for each other, one's loads under another's fold, and sending
+// every load first only brings their folds together.  One ahead / several, us,
+// weights not in the caches: bf16 2048 x 2048 / 4096 / 8192 6.8 / 6.5, 10.1 / 9.4,
+// 16.1 / 14.5; f32 2048 x 2048 / 5120 8.1 / 7.3, 15.2 / 11.7; bf16 3000 x 4096
+// 10.8 / 11.4, 5120 x 2048 8.0 / 8.9, 8192 x 4096 14.9 / 17.7, 32,768 x 5120 55.2 /
+// 55.8, 50,000 x 2048 40.6 / 38.3, 151,936 x 2048 116 / 110; f32 launches of many
+// work-groups draw (20,000 x 4096 54.4 / 54.4).  Of a matrix that is already in
+// L2 several chunks cost the few work-groups up to 0.3 us (bf16 64 x 3072 5.65 /
+// 5.95).  Rows of fewer chunks have nothing to keep in flight (f32 2048 x 1500 6.7 /
+// 6.9).  Off the 16 bytes half rows gain alike (bf16 2048 x 4100 11.5 / 10.0), rows
+// of f32 do not (2048 x 2050 9.1 / 9.4).
+static bool float_ring(int dtype, bool vec, size_t cols, size_t groups) {
   const size_t nchunks = (cols / 8 * 8 + FK - 1) / FK;
-  const int ns = dtype == F32 ? 2 : 4;
-  if (nchunks < (size_t)ns) return 1;
-  return groups < 512 || (dtype != F32 && nchunks == 4) ? ns : 1;
+  if (nchunks < 4 || (!vec && dtype == F32)) return false;
+  return groups <= 256 || (vec && dtype != F32 && groups >= 6144);
 }
 
 hipError_t launch_gemv_float(int dtype, const void* w, const float* x, size_t rows, size_t cols,
                              float* out, hipStream_t st) {
-  return launch_gemv_float_many(dtype, 1, &w, x, &rows, cols, &out, st);
+  if (rows == 0) return hipSuccess;
+  if (rows > (size_t)INT32_MAX - FR || cols > (size_t)INT32_MAX - FK) return hipErrorInvalidValue;
+  if ((uintptr_t)x % 16) return hipErrorInvalidValue;  // x is read in 16-byte pieces
+  const int esz = dtype == F32 ? 4 : 2;
+  const bool vec = (cols * esz) % 16 == 0 && (uintptr_t)w % 16 == 0;
+  const unsigned groups = (unsigned)((rows + FR - 1) / FR);
+  auto run = [&](auto kernel) {
+    return launch(kernel, groups, 256, 0, st, (const uint8_t*)w, x, (int)rows, (int)cols, out);
+  };
+#define HALE_FLOAT_CASE(D)                                                                       \
+  if (dtype == D) {                                                                              \
+    constexpr int NS = D == F32 ? 2 : 4;                                                         \
+    if (float_ring(D, vec, cols, groups))                                                        \
+      return vec ? run(k_gemv_float<D, true, NS>) : run(k_gemv_float<D, D == F32, NS>);          \
+    return vec ? run(k_gemv_float<D, true, 1>) : run(k_gemv_float<D, false, 1>);                 \
+  }
+  HALE_FLOAT_CASE(F32)
+  HALE_FLOAT_CASE(F16)
+  HALE_FLOAT_CASE(BF16)
+#undef HALE_FLOAT_CASE
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemv_float_many(int dtype, int n, const void* const* w, const float* x, const size_t* rows,
@@ -322,16 +354,16 @@ hipError_t launch_gemv_float_many(int dtype, int n, const void* const* w, const 
   }
   if (groups == 0) return hipSuccess;
   auto run = [&](auto kernel) { return launch(kernel, (unsigned)groups, 256, 0, st, m, x, (int)cols); };
-  const bool ring = float_ring(dtype, cols, groups) > 1;
-#define HALE_FLOAT_RING(D, V, M) (ring ? run(k_gemv_float<D, V, M, D == F32 ? 2 : 4>) : run(k_gemv_float<D, V, M, 1>))
-#define HALE_FLOAT_CASE(D)                                                                      \
-  if (dtype == D)                                                                               \
-    return vec ? (n > 1 ? HALE_FLOAT_RING(D, true, true) : HALE_FLOAT_RING(D, true, false))     \
-               : (n > 1 ? HALE_FLOAT_RING(D, false, true) : HALE_FLOAT_RING(D, false, false));
+#define HALE_FLOAT_CASE(D)                                                                            \
+  if (dtype == D) {                                                                                   \
+    constexpr int NS = D == F32 ? 2 : 4;                                                              \
+    if (float_ring(D, vec, cols, groups))                                                             \
+      return vec ? run(k_gemv_float_many<D, true, NS>) : run(k_gemv_float_many<D, D == F32, NS>);     \
+    return vec ? run(k_gemv_float_many<D, true, 1>) : run(k_gemv_float_many<D, false, 1>);            \
+  }
   HALE_FLOAT_CASE(F32)
   HALE_FLOAT_CASE(F16)
   HALE_FLOAT_CASE(BF16)
-#undef HALE_FLOAT_RING
 #undef HALE_FLOAT_CASE
   return hipErrorInvalidValue;
 }

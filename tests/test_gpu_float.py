@@ -51,6 +51,20 @@ def test_float_matvec_bit_exact(ctx, dtype, rows, cols):
 
 
 @pytest.mark.parametrize("dtype", FLOATS)
+@pytest.mark.parametrize("rows,cols", [
+    (37, 1500), (37, 2048), (37, 2052), (37, 2560), (61, 3600), (40, 3072), (30, 4616), (30, 5632), (40, 6704),
+    (33, 3700), (2047, 2500), (20, 6001),  # rows off the 16 bytes
+    (2048, 2048), (2049, 2048),    # 256 work-groups, 257
+    (4100, 2600),
+    (49144, 2056), (49145, 2056),  # 6143 work-groups, 6144: half rows with several chunks in flight again
+])
+def test_float_matvec_chunks_in_flight(ctx, dtype, rows, cols):
+    """Three to fourteen chunks of 512 columns, whole and partial, rows with a
+    tail, and both sides of the lines between one chunk ahead and several."""
+    check_matvec(ctx, dtype, rows, cols, seed=rows * 5 + cols).close()
+
+
+@pytest.mark.parametrize("dtype", FLOATS)
 def test_float_matvec_lm_head_shape(ctx, dtype):
     # a vocabulary-sized output (Qwen3's 151936 rows) over hidden 2048
     check_matvec(ctx, dtype, 151936, 2048, seed=77)
