@@ -225,6 +225,11 @@ hipError_t launch_gemv(int dtype, int epi, const GemvArgs& a, int groups, int sl
                        hipStream_t st);
 hipError_t launch_block_sums(int dtype, const uint8_t* codes, const ActBlock* act, size_t rows,
                              size_t cols, int32_t* isums, hipStream_t st);
+// Whether a conversion of so many pieces (16 bytes of f32 each) gives a thread
+// four of them: where that leaves a work-group of 256 for every CU (bf16, four /
+// one: encoding 100 x 512 3.0 / 2.4 us, 1000 x 1024 3.2 / 2.9, 500 x 4096 3.65
+// with four; one value per thread took 2.5, 3.1, 4.1).
+inline bool convert_wide(size_t pieces) { return pieces >= 256 * 1024; }
 hipError_t launch_fill(float* p, size_t n, float v, hipStream_t st);
 hipError_t launch_copy(void* dst, const void* src, size_t n16, hipStream_t st);
 // n 32-bit words between 16-byte aligned buffers

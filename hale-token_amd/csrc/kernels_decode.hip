@@ -127,26 +127,31 @@ __global__ __launch_bounds__(256) void k_decode_ref(const uint8_t* __restrict__ 
 }
 
 // The same for a source aligned to its element or scale (2 or 4 bytes) and a
-// 16-byte aligned output: 16-byte stores, CONV_U pieces per thread in flight.
-// A piece is 4 values, for q4_0 the 4 + 4 whose codes share four bytes.
-// HBM-bound by the f32 side; 4096 x 14336 q4_0: 105 us with one value per
-// thread, 40 us so.
-constexpr int CONV_U = 4;
-
-template <int DT>
+// 16-byte aligned output: 16-byte stores, U pieces per thread in flight.  A piece
+// is 4 values, for q4_0 the 4 + 4 whose codes share four bytes; the last n % 4
+// values of a float format go to the first threads of the launch (one of their
+// own costs 2.3 us).  HBM-bound by the f32 side; 4096 x 14336 q4_0: 105 us with
+// one value per thread, 40 us so.
+template <int DT, int U>
 __global__ __launch_bounds__(256) void k_decode_vec(const uint8_t* __restrict__ src, size_t n,
                                                     float* __restrict__ out) {
   constexpr int PER = DT == Q4_0 ? 8 : 4;  // values per piece
   const size_t pieces = n / PER;
-  const size_t p0 = (size_t)blockIdx.x * (256 * CONV_U) + threadIdx.x;
+  const size_t last = pieces * PER + threadIdx.x;
+  if ((DT == F32 || DT == F16 || DT == BF16) && blockIdx.x == 0 && last < n) {
+    if constexpr (DT == F32) out[last] = __uint_as_float(((const unsigned*)src)[last]);
+    if constexpr (DT == F16) out[last] = h2f_quiet(((const uint16_t*)src)[last]);
+    if constexpr (DT == BF16) out[last] = __uint_as_float((unsigned)((const uint16_t*)src)[last] << 16);
+  }
+  const size_t p0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x;
   // the piece's codes or elements, loaded whole at their own alignment
   constexpr int WORDS = DT == F32 ? 4 : (DT == F16 || DT == BF16 ? 2 : 1);
   struct __attribute__((packed, aligned(DT == F32 ? 4 : 2))) Words {
     unsigned w[WORDS];
-  } ws[CONV_U];
-  uint16_t sc[CONV_U];
+  } ws[U];
+  uint16_t sc[U];
 #pragma unroll
-  for (int u = 0; u < CONV_U; u++) {  // clamped: unconditional loads stay in flight together
+  for (int u = 0; u < U; u++) {  // clamped: unconditional loads stay in flight together
     const size_t p = p0 + 256 * u < pieces ? p0 + 256 * u : pieces - 1;
     if constexpr (DT == Q8_0 || DT == Q4_0) {
       constexpr int PPB = QK / PER, BB = DT == Q8_0 ? 34 : 18;
@@ -158,7 +163,7 @@ __global__ __launch_bounds__(256) void k_decode_vec(const uint8_t* __restrict__ 
     }
   }
 #pragma unroll
-  for (int u = 0; u < CONV_U; u++) {
+  for (int u = 0; u < U; u++) {
     const size_t p = p0 + 256 * u;
     if (p >= pieces) break;
     const unsigned w = ws[u].w[0];
@@ -2514,22 +2519,21 @@ hipError_t launch_unpack(int dtype, const uint8_t* codes, const uint16_t* scales
 hipError_t launch_decode_ref(int dtype, const void* src, size_t n, float* out, hipStream_t st) {
   if (n == 0) return hipSuccess;
   const uint8_t* b = (const uint8_t*)src;
-  // whole pieces by 16-byte stores; what is left and other alignments value
-  // by value
+  // pieces of 16-byte stores, other alignments value by value
   const size_t per = dtype == Q4_0 ? 8 : 4;
   if (n >= per && (uintptr_t)src % (dtype == F32 ? 4 : 2) == 0 && (uintptr_t)out % 16 == 0) {
-    const size_t done = n / per * per;
-    const unsigned grid = blocks_for(done / per, 256 * CONV_U);
-    hipError_t e = hipErrorInvalidValue;
-    if (dtype == F32) e = launch(k_decode_vec<F32>, grid, 256, 0, st, b, done, out);
-    if (dtype == F16) e = launch(k_decode_vec<F16>, grid, 256, 0, st, b, done, out);
-    if (dtype == BF16) e = launch(k_decode_vec<BF16>, grid, 256, 0, st, b, done, out);
-    if (dtype == Q8_0) e = launch(k_decode_vec<Q8_0>, grid, 256, 0, st, b, done, out);
-    if (dtype == Q4_0) e = launch(k_decode_vec<Q4_0>, grid, 256, 0, st, b, done, out);
-    if (e != hipSuccess || done == n) return e;
-    b += (dtype == F32 ? 4 : 2) * done;  // only float formats leave a remainder
-    out += done;
-    n -= done;
+    const size_t pieces = n / per;
+#define HALE_DECODE_VEC(D)                                                                              \
+  if (dtype == D)                                                                                       \
+    return convert_wide(pieces) ? launch(k_decode_vec<D, 4>, blocks_for(pieces, 256 * 4), 256, 0, st, b, n, out) \
+                                : launch(k_decode_vec<D, 1>, blocks_for(pieces, 256), 256, 0, st, b, n, out);
+    HALE_DECODE_VEC(F32)
+    HALE_DECODE_VEC(F16)
+    HALE_DECODE_VEC(BF16)
+    HALE_DECODE_VEC(Q8_0)
+    HALE_DECODE_VEC(Q4_0)
+#undef HALE_DECODE_VEC
+    return hipErrorInvalidValue;
   }
   const unsigned grid = blocks_for(n, 256);
 #define HALE_DECODE_REF(D) \

@@ -239,7 +239,7 @@ __device__ __forceinline__ uint16_t encode_half(float f) {
   }
 }
 
-// One value per thread: any alignment, and the last n % 4.
+// One value per thread: any alignment.
 template <int DT>
 __global__ __launch_bounds__(256) void k_encode_half(const float* __restrict__ v, size_t n,
                                                      uint16_t* __restrict__ out) {
@@ -247,18 +247,20 @@ __global__ __launch_bounds__(256) void k_encode_half(const float* __restrict__ v
   if (i < n) out[i] = encode_half<DT>(v[i]);
 }
 
-// Four values per thread and step (values 16-byte, out 8-byte aligned),
-// HALF_U steps in flight.
-constexpr int HALF_U = 4;
-template <int DT>
-__global__ __launch_bounds__(256) void k_encode_half4(const float* __restrict__ v, size_t pieces,
+// Four values per thread and step (values 16-byte, out 8-byte aligned), U steps
+// in flight; the last n % 4 by the first threads of the launch.
+template <int DT, int U>
+__global__ __launch_bounds__(256) void k_encode_half4(const float* __restrict__ v, size_t n,
                                                       uint16_t* __restrict__ out) {
-  const size_t p0 = (size_t)blockIdx.x * (256 * HALF_U) + threadIdx.x;
-  f32x4 x[HALF_U];
+  const size_t pieces = n / 4;
+  const size_t p0 = (size_t)blockIdx.x * (256 * U) + threadIdx.x;
+  const size_t last = pieces * 4 + threadIdx.x;
+  if (blockIdx.x == 0 && last < n) out[last] = encode_half<DT>(v[last]);
+  f32x4 x[U];
 #pragma unroll
-  for (int u = 0; u < HALF_U; u++) x[u] = ((const f32x4*)v)[p0 + 256 * u < pieces ? p0 + 256 * u : pieces - 1];
+  for (int u = 0; u < U; u++) x[u] = ((const f32x4*)v)[p0 + 256 * u < pieces ? p0 + 256 * u : pieces - 1];
 #pragma unroll
-  for (int u = 0; u < HALF_U; u++) {
+  for (int u = 0; u < U; u++) {
     const size_t p = p0 + 256 * u;
     if (p >= pieces) break;
     uint64_t w = 0;
@@ -273,14 +275,11 @@ hipError_t launch_encode_half(int dtype, const float* values, size_t n, void* ou
   if (dtype != F16 && dtype != BF16) return hipErrorInvalidValue;
   uint16_t* o = (uint16_t*)out;
   if (n >= 4 && (uintptr_t)values % 16 == 0 && (uintptr_t)out % 8 == 0) {
-    const size_t pieces = n / 4;
-    const unsigned grid = (unsigned)((pieces + 256 * HALF_U - 1) / (256 * HALF_U));
-    const hipError_t e = dtype == F16 ? launch(k_encode_half4<F16>, grid, 256, 0, st, values, pieces, o)
-                                      : launch(k_encode_half4<BF16>, grid, 256, 0, st, values, pieces, o);
-    if (e != hipSuccess || n % 4 == 0) return e;
-    values += 4 * pieces;
-    o += 4 * pieces;
-    n %= 4;
+    const bool wide = convert_wide(n / 4);
+    const unsigned per = wide ? 1024 : 256, grid = (unsigned)((n / 4 + per - 1) / per);
+    auto run = [&](auto kernel) { return launch(kernel, grid, 256, 0, st, values, n, o); };
+    if (dtype == F16) return wide ? run(k_encode_half4<F16, 4>) : run(k_encode_half4<F16, 1>);
+    return wide ? run(k_encode_half4<BF16, 4>) : run(k_encode_half4<BF16, 1>);
   }
   const unsigned grid = (unsigned)((n + 255) / 256);
   return dtype == F16 ? launch(k_encode_half<F16>, grid, 256, 0, st, values, n, o)

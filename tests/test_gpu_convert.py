@@ -150,6 +150,14 @@ def test_device_conversions_at_any_size_and_offset(ctx, dtype, n, in_off, out_of
         b.free()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("n", [1048574, 1048576, 1048579, 2097120, 2097184])
+def test_device_conversions_one_or_four_pieces_a_thread(ctx, dtype, n):
+    """Both sides of the sizes from which a thread takes four pieces, with
+    one to three values after the last."""
+    test_device_conversions_at_any_size_and_offset(ctx, dtype, n, 0, 0)
+
+
 def test_decode_rejects_ragged_quantized_rows(ctx):
     """Q8_0 / Q4_0 rows must hold whole blocks (DType::row_bytes)."""
     src, out = np.zeros(64, np.uint8), np.zeros(48, np.float32)
