@@ -117,8 +117,11 @@ struct DownArgs {
   // routes or combine): x (f32, 16-byte aligned) quantized by the kernel,
   // or hact when null
   const float* x;
-  // launch_matvec_many: further matrices of the same row length and x;
-  // work-groups from more[i].first on take matrix i + 1
+};
+
+// launch_matvec_many: further matrices of the same row length and x; work-groups
+// from more[i].first on take matrix i + 1.
+struct DownManyArgs : DownArgs {
   struct {
     const uint8_t* codes;
     const uint16_t* scales;

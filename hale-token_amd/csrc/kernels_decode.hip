@@ -1708,8 +1708,9 @@ static inline size_t down_tile_lds(int slots, int nb) { return (size_t)slots * n
 // (S = 1, no routes): out[row] is the row's sum; x, when given, is
 // quantized into the staging by the work-group (the expressions of
 // k_act_quant, so the same q8 blocks).
-template <int DT, int S, int NW, int RW, int UPW, bool PLAIN = false>
-__global__ __launch_bounds__(64 * NW) void k_down_tile(DownArgs a) {
+// ARGS: DownManyArgs where a launch may hold several matrices (launch_spread).
+template <int DT, int S, int NW, int RW, int UPW, bool PLAIN = false, class ARGS = DownArgs>
+__global__ __launch_bounds__(64 * NW) void k_down_tile(ARGS a) {
   constexpr int CH = Layout<DT>::CH;
   constexpr int LPS = S == 1 ? 64 : 32;  // lanes per slot
   constexpr int BPL = LPS / RW;       // blocks per slot and wave-load
@@ -1784,7 +1785,7 @@ __global__ __launch_bounds__(64 * NW) void k_down_tile(DownArgs a) {
   // tile's scale lines).
   constexpr int PER_TILE = 32 / RW;
   int g = blockIdx.x, groups = gridDim.x;
-  if constexpr (PLAIN) {  // of several matrices, this work-group's
+  if constexpr (std::is_same_v<ARGS, DownManyArgs>) {  // of several matrices, this work-group's
     if (a.more[0].codes) {  // uniform
       const int second = a.more[0].first, third = a.more[1].codes ? a.more[1].first : groups;
       const int m = g < second ? 0 : (g < third ? 1 : 2);
@@ -2863,9 +2864,15 @@ static bool matvec_spread(int nb, size_t rows) {
 bool matvec_takes_x(int nb, size_t rows) { return nb <= MATVEC_XQ_MAX_NB || matvec_spread(nb, rows); }
 
 // k_down_tile's plain form over n matrices of one row length and x; rows per
-// work-group as for one matrix of all their rows.
+// work-group as for one matrix of all their rows.  One matrix on 32-row
+// work-groups has arguments without the others', which cost it 1 to 3 % (14,336 x
+// 4096 q8_0 11.9 against 11.6 us, q4_0 8.7 / 8.5; 8192 x 8192 q8_0 13.9 / 13.7).  On
+// 16-row work-groups it keeps them: the kernel that may hold several starts its
+// weight loads later, behind x, which measured mostly faster there (4096 x 4096 not in the
+// caches, q8_0 7.2 against 7.5, q4_0 6.3 / 6.6; 2048 x 4096 6.4 / 6.6, 2048 x 2048
+// 5.2 / 5.0).
 static hipError_t launch_spread(int dtype, int n, const MatvecArgs* a, hipStream_t st) {
-  DownArgs d{};
+  DownManyArgs d{};
   d.codes = a[0].codes;
   d.scales = a[0].scales;
   d.nb = a[0].nb;
@@ -2886,10 +2893,15 @@ static hipError_t launch_spread(int dtype, int n, const MatvecArgs* a, hipStream
   }
   const dim3 grid((unsigned)(prow / (half ? 16 : 32)));
   const uint32_t lds = (uint32_t)down_tile_lds(1, d.nb);
-  if (half && dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 16, 1, true>, grid, 1024, lds, st, d);
-  if (half) return launch(k_down_tile<Q4_0, 1, 16, 16, 2, true>, grid, 1024, lds, st, d);
-  if (dtype == Q8_0) return launch(k_down_tile<Q8_0, 1, 16, 32, 1, true>, grid, 1024, lds, st, d);
-  return launch(k_down_tile<Q4_0, 1, 16, 32, 2, true>, grid, 1024, lds, st, d);
+  if (half)
+    return dtype == Q8_0 ? launch(k_down_tile<Q8_0, 1, 16, 16, 1, true, DownManyArgs>, grid, 1024, lds, st, d)
+                         : launch(k_down_tile<Q4_0, 1, 16, 16, 2, true, DownManyArgs>, grid, 1024, lds, st, d);
+  if (n > 1)
+    return dtype == Q8_0 ? launch(k_down_tile<Q8_0, 1, 16, 32, 1, true, DownManyArgs>, grid, 1024, lds, st, d)
+                         : launch(k_down_tile<Q4_0, 1, 16, 32, 2, true, DownManyArgs>, grid, 1024, lds, st, d);
+  const DownArgs& one = d;
+  return dtype == Q8_0 ? launch(k_down_tile<Q8_0, 1, 16, 32, 1, true>, grid, 1024, lds, st, one)
+                       : launch(k_down_tile<Q4_0, 1, 16, 32, 2, true>, grid, 1024, lds, st, one);
 }
 
 // The spread form's shapes, for each matrix alone and for their rows together
