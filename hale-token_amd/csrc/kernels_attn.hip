@@ -4,15 +4,18 @@
 // src/model/kv_cache.rs).
 //
 // Every sum keeps the reference's order, so every result is bit-identical:
-//   - RMSNorm's sum of squares runs in order from -0.0 (Iterator::sum), then
+//   - RMSNorm's squares are summed in order (from -0.0 in the reference,
+//     Iterator::sum; the start shows only without values), then
 //     1 / sqrt(sum / n + eps), then x * scale * w (rms_norm) or
 //     x * (scale * w) (rms_norm_in_place);
 //   - a score is the in-order sum q[0]k[0] + q[1]k[1] + ... from -0.0,
 //     times 1 / sqrt(hd); softmax is softmax_in_place (max, glibc exp, an
 //     in-order sum from 0.0, one division per score);
 //   - a context element is 0 + p_0 v_0 + p_1 v_1 + ... in position order.
-// The products and the exponentials are computed in parallel; each
-// sequential sum runs in one lane.
+// The products and the exponentials are computed in parallel.  The sums of
+// RMSNorm and, in rows of up to 8192 positions, of softmax are formed by many
+// lanes with the chain's bits (ordered_sum.h); scores, the context, QK-norm and
+// the softmax of longer rows are chains, one lane each.
 #pragma clang fp contract(off)
 
 #include "hale_device.h"
