@@ -2599,21 +2599,24 @@ hipError_t launch_route_logits(const float* router, const float* x, int H, int E
   if (H > ROUTE_MAX_H || E > ROUTE_MAX_E || H % QK || E < 1 || T < 1) return hipErrorInvalidValue;
   if (T >= ROUTE_TILED_MIN_T) {
     // many tokens: tiles of router rows and tokens, the activation blocks
-    // quantized by the same launch.  Eight experts x 8 tokens, a logit per
-    // lane, while two of them per CU (what their LDS allows) take the whole
-    // call at once: 128 experts, 256 tokens (512 work-groups) 13.1 us at H
-    // 2048 and 19.7 at H 4096, with 16 x 16 tiles 16.8 and 27.5; 257 tokens
-    // 18.8 and 29.8 against 17.1 and 27.6, 600 tokens 26.1 and 43.5 against
-    // 23.8 and 39.4.  16 x 16 beyond, two experts x two tokens per lane (2048
-    // tokens x 128 experts 44.0 and 80.2 us, 68.3 and 124 with 8 x 8), but
-    // 8 x 8 at any length for up to 8 experts, of whose 16-row tile half is
-    // padding (H 4096, 2056 / 4096 / 8192 tokens: 34.3 / 39.6 / 75.3 us
-    // against 48.4 / 52.4 / 79.6), and for up to 32 experts until 16 x 16 tiles
-    // come to three quarters of the CUs (H 4096, 16 experts x 2056 / 3000 / 4096
-    // tokens, 129 / 188 / 256 tiles: 41.3 / 45.0 / 55.4 against 48.6 / 49.3 /
-    // 52.8; 64 experts draw there).
+    // quantized by the same launch.  A logit per lane while that takes one
+    // round: 8 experts x 8 tokens up to a work-group per CU, then 16 x 8, which
+    // stages a token's row half as often (128 experts, 128 / 160 / 256 tokens at
+    // H 4096 17.1 / 19.8 / 20.8 us with 8 x 8, 19.0 / 19.3 / 19.9 with 16 x 8).
+    // 16 x 16 beyond, two experts x two tokens per lane (128 experts, 256 / 257 /
+    // 2048 tokens 27.5 / 27.6 / 80 us, with 8 x 8 20.8 / 29.8 / 124).  8 x 8 also
+    // where two per CU, what their LDS allows, take the call and 16 x 8 would
+    // not; at any length for up to 8 experts, of whose 16-row tile half is padding
+    // (H 4096, 2056 / 4096 / 8192 tokens: 34.3 / 39.6 / 75.3 us against 48.4 /
+    // 52.4 / 79.6 with 16 x 16); and for up to 32 experts until 16 x 16 tiles come
+    // to three quarters of the CUs (16 experts x 2056 / 3000 / 4096 tokens, 129 /
+    // 188 / 256 tiles: 41.3 / 45.0 / 55.4 against 48.6 / 49.3 / 52.8; 64 experts
+    // draw there).
     const int et8 = (E + 7) / 8, tt8 = (T + 7) / 8, et = (E + 15) / 16, tt = (T + 15) / 16;
-    if ((size_t)et8 * tt8 <= 512 || (E <= 8 && tt8 <= 0xffff) || (E <= 32 && et * tt < 192))
+    const size_t n8 = (size_t)et8 * tt8;
+    if (n8 > 256 && (size_t)et * tt8 <= 256)
+      return launch(k_route_logits_tiled<16, 1, 1, 64>, dim3(et, tt8), 1024, 0, st, router, x, H, E, T, logits, act);
+    if (n8 <= 512 || (E <= 8 && tt8 <= 0xffff) || (E <= 32 && et * tt < 192))
       return launch(k_route_logits_tiled<8, 1, 1, 64>, dim3(et8, tt8), 512, 0, st, router, x, H, E, T, logits, act);
     return launch(k_route_logits_tiled<16, 2, 2, 32>, dim3(et, tt), 512, 0, st, router, x, H, E, T, logits, act);
   }

@@ -95,15 +95,18 @@ def test_grouped_router_many_tokens(ctx, dtype, Hd, I, E, k, T):
     (H.Q4_0, 288, 32, 1000, 2, 49),   # 63 x 4 tiles
     (H.Q8_0, 4128, 32, 128, 4, 241),  # a partial chunk (516 steps)
     (H.Q8_0, 512, 32, 128, 4, 240),
-    (H.Q8_0, 512, 32, 128, 4, 256),   # 512 tiles of 8 x 8
-    (H.Q8_0, 512, 32, 128, 4, 257),   # 528 of them: 16 x 16
+    (H.Q8_0, 512, 32, 128, 4, 128),   # 256 tiles of 8 x 8
+    (H.Q8_0, 288, 32, 123, 4, 133),   # 272 of them: 16 x 8, partial expert and token tiles
+    (H.Q8_0, 512, 32, 128, 4, 256),   # 256 tiles of 16 x 8
+    (H.Q8_0, 512, 32, 128, 4, 257),   # 264 of them: 16 x 16
+    (H.Q4_0, 288, 32, 40, 2, 717),    # 270 of 16 x 8, 450 of 8 x 8: those
     (H.Q4_0, 288, 32, 7, 2, 4105),    # up to 8 experts: 8 x 8 at any length
     (H.Q8_0, 288, 32, 24, 2, 1520),   # 2 x 95 tiles of 16 x 16, below three quarters of the CUs: 8 x 8
     (H.Q8_0, 288, 32, 24, 2, 1530),   # 2 x 96: 16 x 16, half of the last expert tile padding
 ])
 def test_grouped_router_register_tiles(ctx, dtype, Hd, I, E, k, T):
-    """The router's tiles: 8 x 8, a logit per lane, or 16 x 16, two experts x
-    two tokens per lane, on both sides of each line between them."""
+    """The router's tiles: 8 x 8 and 16 x 8, a logit per lane, or 16 x 16, two
+    experts x two tokens per lane, on both sides of each line between them."""
     L = O.OracleMoe.synthetic(dtype, Hd, I, E, k, normalize_topk=True, seed=Hd + E + T, with_router=True)
     moe = make_layer(ctx, L)
     check(moe, L, O.normal(T + Hd, T * Hd).reshape(T, Hd))
